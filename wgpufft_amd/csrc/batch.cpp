@@ -48,7 +48,7 @@ static std::string batch_reject_reason(const Plan& p) {
         bool ok = false;
         switch (op->kind) {
             case OP_REG: ok = batch_class_for(op->rv) >= 0; break;
-            case OP_LDS: ok = batch_lds_class(op->prec, op->ldm, op->stm, op->post) >= 0; break;
+            case OP_LDS: ok = batch_lds_class(op->prec, op->ldm, op->stm, op->post, op->mix.ns > 0) >= 0; break;
             case OP_RADER:
             case OP_BLUESTEIN:
             case OP_CHIRP_PRE:
@@ -212,12 +212,20 @@ void batch_build(const BatchEntry* entries, int32_t count, char* ws_base, BatchB
                     unit = op.rv->n;
                     break;
                 case OP_LDS:
-                    cls = (uint32_t)batch_lds_class(op.prec, op.ldm, op.stm, op.post);
+                    cls = (uint32_t)batch_lds_class(op.prec, op.ldm, op.stm, op.post, op.mix.ns > 0);
                     d.a = op.a;
                     d.sc = op.sc;
-                    lpw = op.sc.lpw;
-                    op_lds = lds_kernel_bytes(op.prec, op.sc.n, op.sc.lpw);
-                    unit = op.sc.n;
+                    d.mix = op.mix;
+                    // a plan made for one line: the tile for all lines that run it
+                    if (op.mix.ns && e.mult > 1) {
+                        Mix m;
+                        if (mix_plan(P.arith, op.n, (uint64_t)op.a.lines * e.mult, op.ld_lf, op.st_lf, P.lds_budget, 256,
+                                     0, &m))
+                            d.mix = m;
+                    }
+                    lpw = d.mix.ns ? d.mix.lpw : op.sc.lpw;
+                    op_lds = d.mix.ns ? mix_lds_bytes(P.arith, d.mix) : lds_kernel_bytes(op.prec, op.sc.n, op.sc.lpw);
+                    unit = op.n;
                     break;
                 case OP_RADER:
                 case OP_BLUESTEIN:

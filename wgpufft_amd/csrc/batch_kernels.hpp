@@ -60,6 +60,11 @@ enum BatchClass : uint32_t {
     BC_REGB_8192,
     // fused Rader convolution with medium prime radices (17..61), f32
     BC_RADER_MED,
+    // complex lines of a runtime schedule (mix_kernels.hpp)
+    BC_MIX,
+    BC_MIX_POST,
+    BC_MIX_F64,
+    BC_MIX_POST_F64,
     BC_COUNT
 };
 
@@ -80,7 +85,8 @@ struct BatchTile {
 // Arguments of one op of one transform, device pointers already bound.
 struct OpDesc {
     LineArgs a;   // line ops (register and LDS classes)
-    Sched sc;     // LDS classes
+    Sched sc;     // LDS classes of real lines
+    Mix mix;      // LDS classes of complex lines
     ConvArgs conv;  // Rader / Bluestein classes; element-wise classes (io, chirp, filt, n, m)
 };
 
@@ -88,8 +94,8 @@ struct OpDesc {
 // complex in and out), or -1.
 int batch_class_for(const RegVariant* v);
 // Class of a runtime-schedule LDS op (precision, load/store modes, twiddle on
-// store), or -1.
-int batch_lds_class(int prec, int ldm, int stm, int post);
+// store, register form), or -1.
+int batch_lds_class(int prec, int ldm, int stm, int post, bool mix);
 
 hipError_t launch_batch(const BatchTile* tiles, uint32_t ntiles, uint32_t* counter, const OpDesc* ops,
                         uint32_t grid, size_t lds_bytes, hipStream_t s);

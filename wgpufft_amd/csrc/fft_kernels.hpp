@@ -73,8 +73,8 @@ __device__ __forceinline__ LineBase line_base(const LineArgs& a, uint32_t g) {
 
 // W_P^t as the FP64 product of two FP64 table entries.
 __device__ __forceinline__ double2 post_f64(const LineArgs& a, uint64_t t) {
-    const double2 h = a.post_hi[t >> a.post_shift];
-    const double2 l = a.post_lo[t & a.post_mask];
+    const vd2_t h = gptr<vd2_t>(a.post_hi)[t >> a.post_shift];
+    const vd2_t l = gptr<vd2_t>(a.post_lo)[t & a.post_mask];
     return make_double2(h.x * l.x - h.y * l.y, h.x * l.y + h.y * l.x);
 }
 
@@ -209,7 +209,7 @@ template <class Fmt, bool NT = true>
 __device__ __forceinline__ void load_pair_at(const LineArgs& a, uint32_t i, cpx<typename Fmt::T>& v0,
                                              cpx<typename Fmt::T>& v1) {
     if constexpr (Fmt::kId == 0) {
-        const vf4_t* q4 = reinterpret_cast<const vf4_t*>(reinterpret_cast<const float2*>(a.in) + i);
+        const auto* q4 = (const MIFFT_GLOBAL vf4_t*)(gptr<vf2_t>(a.in) + i);
         vf4_t q;
         if constexpr (NT) q = __builtin_nontemporal_load(q4);
         else q = *q4;
@@ -242,7 +242,7 @@ __device__ __forceinline__ void store_pair_at(const LineArgs& a, uint32_t i, uin
     v0 = mk<T>(v0.x * s.re, v0.y * s.im);
     v1 = mk<T>(v1.x * s.re, v1.y * s.im);
     if constexpr (Fmt::kId == 0) {
-        *reinterpret_cast<float4*>(reinterpret_cast<float2*>(a.out) + i) = make_float4(v0.x, v0.y, v1.x, v1.y);
+        *(MIFFT_GLOBAL vf4_t*)(gptr<vf2_t>(a.out) + i) = vf4_t{v0.x, v0.y, v1.x, v1.y};
     } else {
         Fmt::st(a.out, i, v0);
         Fmt::st(a.out, i + 1, v1);
@@ -772,7 +772,7 @@ __device__ __forceinline__ void lds_stage(const cpx<T>* src, cpx<T>* dst, uint32
         for (int m = 0; m < R; m++) w[m] = s[lpad(j + m * nr)];
         if (L > 1) {
 #pragma unroll
-            for (int m = 1; m < R; m++) w[m] = cmul(w[m], ld_tw<T>(tw, twoff + (m - 1) * L + k));
+            for (int m = 1; m < R; m++) w[m] = cmul(w[m], ld_tw_any<T>(tw, twoff + (m - 1) * L + k));
         }
         Dft<R, T>::run(w);
         cpx<T>* d = dst + l * lstr;
@@ -817,8 +817,8 @@ __device__ __forceinline__ void prime_in(cpx<T>* ap, cpx<T>* am, cpx<T>& sum, co
     if constexpr (m <= (R - 1) / 2) {
         cpx<T> x = s[lpad(j + m * nr)], y = s[lpad(j + (R - m) * nr)];
         if (L > 1) {
-            x = cmul(x, ld_tw<T>(tw, twoff + (m - 1) * L + k));
-            y = cmul(y, ld_tw<T>(tw, twoff + (R - m - 1) * L + k));
+            x = cmul(x, ld_tw_any<T>(tw, twoff + (m - 1) * L + k));
+            y = cmul(y, ld_tw_any<T>(tw, twoff + (R - m - 1) * L + k));
         }
         ap[m - 1] = x + y;
         am[m - 1] = x - y;

@@ -92,25 +92,39 @@ typedef float vf2_t __attribute__((ext_vector_type(2)));
 typedef float vf4_t __attribute__((ext_vector_type(4)));
 typedef double vd2_t __attribute__((ext_vector_type(2)));
 
+// A device-memory pointer as an address-space-1 one.  A pointer that a kernel
+// reads from memory (the batched kernel's descriptors) is generic to the
+// compiler: its loads and stores become FLAT ones, which every LDS wait waits
+// for too.
+#define MIFFT_GLOBAL __attribute__((address_space(1)))
+template <class V>
+__device__ __forceinline__ const MIFFT_GLOBAL V* gptr(const void* p) {
+    return (const MIFFT_GLOBAL V*)p;
+}
+template <class V>
+__device__ __forceinline__ MIFFT_GLOBAL V* gptr(void* p) {
+    return (MIFFT_GLOBAL V*)p;
+}
+
 struct FmtF32 {
     using T = float;
     static constexpr int kId = 0;
     static __device__ __forceinline__ cpx<float> ld(const void* p, uint64_t i) {
-        const vf2_t v = __builtin_nontemporal_load(reinterpret_cast<const vf2_t*>(p) + i);
+        const vf2_t v = __builtin_nontemporal_load(gptr<vf2_t>(p) + i);
         return mk<float>(v.x, v.y);
     }
     static __device__ __forceinline__ cpx<float> ld_c(const void* p, uint64_t i) {
-        const vf2_t v = reinterpret_cast<const vf2_t*>(p)[i];
+        const vf2_t v = gptr<vf2_t>(p)[i];
         return mk<float>(v.x, v.y);
     }
     static __device__ __forceinline__ void st(void* p, uint64_t i, cpx<float> v) {
-        reinterpret_cast<float2*>(p)[i] = make_float2(v.x, v.y);
+        gptr<vf2_t>(p)[i] = vf2_t{v.x, v.y};
     }
     static __device__ __forceinline__ float ld_real(const void* p, uint64_t i) {
-        return reinterpret_cast<const float*>(p)[i];
+        return gptr<float>(p)[i];
     }
     static __device__ __forceinline__ void st_real(void* p, uint64_t i, float v) {
-        reinterpret_cast<float*>(p)[i] = v;
+        gptr<float>(p)[i] = v;
     }
 };
 
@@ -118,21 +132,21 @@ struct FmtF64 {
     using T = double;
     static constexpr int kId = 1;
     static __device__ __forceinline__ cpx<double> ld(const void* p, uint64_t i) {
-        const vd2_t v = __builtin_nontemporal_load(reinterpret_cast<const vd2_t*>(p) + i);
+        const vd2_t v = __builtin_nontemporal_load(gptr<vd2_t>(p) + i);
         return mk<double>(v.x, v.y);
     }
     static __device__ __forceinline__ cpx<double> ld_c(const void* p, uint64_t i) {
-        const vd2_t v = reinterpret_cast<const vd2_t*>(p)[i];
+        const vd2_t v = gptr<vd2_t>(p)[i];
         return mk<double>(v.x, v.y);
     }
     static __device__ __forceinline__ void st(void* p, uint64_t i, cpx<double> v) {
-        reinterpret_cast<double2*>(p)[i] = make_double2(v.x, v.y);
+        gptr<vd2_t>(p)[i] = vd2_t{v.x, v.y};
     }
     static __device__ __forceinline__ double ld_real(const void* p, uint64_t i) {
-        return reinterpret_cast<const double*>(p)[i];
+        return gptr<double>(p)[i];
     }
     static __device__ __forceinline__ void st_real(void* p, uint64_t i, double v) {
-        reinterpret_cast<double*>(p)[i] = v;
+        gptr<double>(p)[i] = v;
     }
 };
 
@@ -148,30 +162,47 @@ struct FmtDF64 {
         return make_float2(hi, lo);
     }
     static __device__ __forceinline__ cpx<double> ld(const void* p, uint64_t i) {
-        const vf4_t v = __builtin_nontemporal_load(reinterpret_cast<const vf4_t*>(p) + i);
+        const vf4_t v = __builtin_nontemporal_load(gptr<vf4_t>(p) + i);
         return mk<double>(join(v.x, v.y), join(v.z, v.w));
     }
     static __device__ __forceinline__ cpx<double> ld_c(const void* p, uint64_t i) {
-        const vf4_t v = reinterpret_cast<const vf4_t*>(p)[i];
+        const vf4_t v = gptr<vf4_t>(p)[i];
         return mk<double>(join(v.x, v.y), join(v.z, v.w));
     }
     static __device__ __forceinline__ void st(void* p, uint64_t i, cpx<double> v) {
         float2 a = split(v.x), b = split(v.y);
-        reinterpret_cast<float4*>(p)[i] = make_float4(a.x, a.y, b.x, b.y);
+        gptr<vf4_t>(p)[i] = vf4_t{a.x, a.y, b.x, b.y};
     }
     static __device__ __forceinline__ double ld_real(const void* p, uint64_t i) {
-        float2 v = reinterpret_cast<const float2*>(p)[i];
+        const vf2_t v = gptr<vf2_t>(p)[i];
         return join(v.x, v.y);
     }
     static __device__ __forceinline__ void st_real(void* p, uint64_t i, double v) {
-        reinterpret_cast<float2*>(p)[i] = split(v);
+        const float2 w = split(v);
+        gptr<vf2_t>(p)[i] = vf2_t{w.x, w.y};
     }
 };
 
 // Twiddle tables are stored in the arithmetic type (cpx<float> for F32,
 // cpx<double> for F64/DF64), each entry rounded once from an FP64 value.
 template <class T>
+struct Vec2;
+template <>
+struct Vec2<float> {
+    using V = vf2_t;
+};
+template <>
+struct Vec2<double> {
+    using V = vd2_t;
+};
+template <class T>
 __device__ __forceinline__ cpx<T> ld_tw(const void* tab, uint32_t i) {
+    const typename Vec2<T>::V v = gptr<typename Vec2<T>::V>(tab)[i];
+    return mk<T>(v.x, v.y);
+}
+// The same from a table that may sit in LDS (small volumes).
+template <class T>
+__device__ __forceinline__ cpx<T> ld_tw_any(const void* tab, uint32_t i) {
     return reinterpret_cast<const cpx<T>*>(tab)[i];
 }
 
@@ -325,6 +356,39 @@ struct DftComp {
     }
 };
 
+// Composite R = R1 * R2 with coprime factors (Good-Thomas): with n = R2 n1 +
+// R1 n2 mod R, W_R^(n k) = W_R1^(n1 k) W_R2^(n2 k), so the two passes need no
+// twiddle between them: the index maps are register names, and (R1 - 1)
+// (R2 - 1) complex multiplies and their rounding go away (radix 15: 32 of 210
+// instructions, radix 10: 16 of 108).
+template <int R1, int R2, class T>
+struct DftCoprime {
+    static constexpr int R = R1 * R2;
+    static constexpr int out(int k1, int k2) {
+        int k = k1;
+        while (k % R2 != k2) k += R1;
+        return k;
+    }
+    static __device__ __forceinline__ void run(cpx<T>* v) {
+        cpx<T> y[R2][R1];
+#pragma unroll
+        for (int n2 = 0; n2 < R2; n2++) {
+#pragma unroll
+            for (int n1 = 0; n1 < R1; n1++) y[n2][n1] = v[(R2 * n1 + R1 * n2) % R];
+            Dft<R1, T>::run(y[n2]);
+        }
+#pragma unroll
+        for (int k1 = 0; k1 < R1; k1++) {
+            cpx<T> z[R2];
+#pragma unroll
+            for (int n2 = 0; n2 < R2; n2++) z[n2] = y[n2][k1];
+            Dft<R2, T>::run(z);
+#pragma unroll
+            for (int k2 = 0; k2 < R2; k2++) v[out(k1, k2)] = z[k2];
+        }
+    }
+};
+
 template <class T>
 struct Dft<8, T> : DftComp<2, 4, T> {};
 template <class T>
@@ -334,17 +398,17 @@ struct Dft<32, T> : DftComp<4, 8, T> {};
 template <class T>
 struct Dft<64, T> : DftComp<8, 8, T> {};
 template <class T>
-struct Dft<6, T> : DftComp<2, 3, T> {};
+struct Dft<6, T> : DftCoprime<2, 3, T> {};
 template <class T>
 struct Dft<9, T> : DftComp<3, 3, T> {};
 template <class T>
-struct Dft<10, T> : DftComp<2, 5, T> {};
+struct Dft<10, T> : DftCoprime<2, 5, T> {};
 template <class T>
-struct Dft<12, T> : DftComp<4, 3, T> {};
+struct Dft<12, T> : DftCoprime<4, 3, T> {};
 template <class T>
-struct Dft<14, T> : DftComp<2, 7, T> {};
+struct Dft<14, T> : DftCoprime<2, 7, T> {};
 template <class T>
-struct Dft<15, T> : DftComp<3, 5, T> {};
+struct Dft<15, T> : DftCoprime<3, 5, T> {};
 
 // ---------------------------------------------------------- fast division
 // floor(x / d) for x < 2^31 with a host-computed magic (m, s):

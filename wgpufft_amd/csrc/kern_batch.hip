@@ -15,6 +15,7 @@
 // This is the gfx950 counterpart of recording many plans into one shared
 // compute pass with FftRecorder (src/plan.rs:38-95, src/runtime/recorder.rs).
 #include "batch_kernels.hpp"
+#include "mix_kernels.hpp"
 #include "reg_conv.hpp"
 
 namespace mifft {
@@ -30,6 +31,18 @@ __device__ __forceinline__ uint32_t claim_tile(uint32_t* counter) {
     return t;
 }
 
+// A pointer argument of a class function (the same in every lane, which the
+// compiler does not know of a function's arguments) as a uniform pointer to
+// memory that the launch does not write: its loads are scalar ones.
+template <class V>
+__device__ __forceinline__ const V* uniform_const(const V* p) {
+    const uint64_t v = (uint64_t)p;
+    // (readfirstlane returns a signed int: each half widens through uint32_t)
+    const uint64_t u = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)v) |
+                       ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(v >> 32)) << 32);
+    return (const V*)(const __attribute__((address_space(4))) V*)u;
+}
+
 // Every class is a separate (not inlined) function: inlined into one switch,
 // the register allocation of the kernel would be the worst path's, and the
 // whole persistent kernel would run at one wave per SIMD.  A call boundary
@@ -43,6 +56,9 @@ __device__ __forceinline__ uint32_t tile_run(const BatchTile* __restrict__ tiles
                                              uint32_t* counter, const OpDesc* __restrict__ ops, uint32_t t,
                                              Body&& body) {
     t = __builtin_amdgcn_readfirstlane(t);
+    ntiles = __builtin_amdgcn_readfirstlane(ntiles);
+    tiles = uniform_const(tiles);
+    ops = uniform_const(ops);
     const uint32_t cls = tiles[t].cls;
     for (;;) {
         const BatchTile tl = tiles[t];
@@ -67,6 +83,12 @@ template <class Fmt, int LDM, int STM, bool POST>
 __device__ __noinline__ uint32_t lds_tiles(MIFFT_TILE_ARGS) {
     return tile_run(tiles, ntiles, counter, ops, t, [&](const OpDesc& d, uint32_t g0) {
         lds_fft_tile<Fmt, LDM, STM, POST>(d.a, d.sc, smem, g0);
+    });
+}
+template <class Fmt, bool POST>
+__device__ __noinline__ uint32_t mix_tiles(MIFFT_TILE_ARGS) {
+    return tile_run(tiles, ntiles, counter, ops, t, [&](const OpDesc& d, uint32_t g0) {
+        mix_tile<Fmt, LD_COMPLEX, ST_COMPLEX, POST>(d.a, d.mix, smem, g0);
     });
 }
 template <class Fmt, bool MED = false>
@@ -125,6 +147,10 @@ __global__ void __launch_bounds__(256, 4) k_batch(const BatchTile* __restrict__ 
             case BC_LDS_C2R: t = lds_tiles<FmtF32, LD_HERMITIAN, ST_REAL, false>(MIFFT_TILE_PASS); break;
             case BC_LDS_F64: t = lds_tiles<FmtF64, LD_COMPLEX, ST_COMPLEX, false>(MIFFT_TILE_PASS); break;
             case BC_LDS_POST_F64: t = lds_tiles<FmtF64, LD_COMPLEX, ST_COMPLEX, true>(MIFFT_TILE_PASS); break;
+            case BC_MIX: t = mix_tiles<FmtF32, false>(MIFFT_TILE_PASS); break;
+            case BC_MIX_POST: t = mix_tiles<FmtF32, true>(MIFFT_TILE_PASS); break;
+            case BC_MIX_F64: t = mix_tiles<FmtF64, false>(MIFFT_TILE_PASS); break;
+            case BC_MIX_POST_F64: t = mix_tiles<FmtF64, true>(MIFFT_TILE_PASS); break;
             case BC_RADER: t = rader_tiles<FmtF32>(MIFFT_TILE_PASS); break;
             case BC_BLUESTEIN: t = bluestein_tiles<FmtF32>(MIFFT_TILE_PASS); break;
             case BC_RADER_F64: t = rader_tiles<FmtF64>(MIFFT_TILE_PASS); break;
@@ -195,14 +221,14 @@ hipError_t launch_batch_reset(uint32_t* counters, uint32_t n, hipStream_t s) {
     return hipGetLastError();
 }
 
-int batch_lds_class(int prec, int ldm, int stm, int post) {
-    if (prec == P_F32) {
-        if (ldm == LD_COMPLEX && stm == ST_COMPLEX) return post ? BC_LDS_POST : BC_LDS;
-        if (!post && ldm == LD_REAL && stm == ST_PACKED) return BC_LDS_R2C;
-        if (!post && ldm == LD_HERMITIAN && stm == ST_REAL) return BC_LDS_C2R;
+int batch_lds_class(int prec, int ldm, int stm, int post, bool mix) {
+    if (ldm == LD_COMPLEX && stm == ST_COMPLEX) {
+        if (prec == P_F32) return mix ? (post ? BC_MIX_POST : BC_MIX) : (post ? BC_LDS_POST : BC_LDS);
+        if (prec == P_F64) return mix ? (post ? BC_MIX_POST_F64 : BC_MIX_F64) : (post ? BC_LDS_POST_F64 : BC_LDS_F64);
         return -1;
     }
-    if (prec == P_F64 && ldm == LD_COMPLEX && stm == ST_COMPLEX) return post ? BC_LDS_POST_F64 : BC_LDS_F64;
+    if (prec == P_F32 && !post && ldm == LD_REAL && stm == ST_PACKED) return BC_LDS_R2C;
+    if (prec == P_F32 && !post && ldm == LD_HERMITIAN && stm == ST_REAL) return BC_LDS_C2R;
     return -1;
 }
 

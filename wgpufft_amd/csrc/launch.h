@@ -65,6 +65,42 @@ hipError_t launch_lds(int prec, int ldm, int stm, int post, const LineArgs& a, c
 size_t lds_kernel_bytes(int prec, uint32_t n, uint32_t lpw);
 constexpr size_t kLdsBudget = 160 * 1024;
 
+// Runtime-schedule register line kernels (mix_kernels.hpp, kern_mix.hip): the
+// schedule and tile shape of one length (mix_plan.cpp).  Counts are in
+// elements; the d* fields are mix_div multipliers.
+constexpr int kMixStages = 8;
+struct MixStage {
+    uint32_t code;      // radix + 32 * unroll
+    uint32_t nr, nrp;   // butterflies per line and their LDS pitch (odd)
+    uint32_t nrp_prev;  // the previous stage's pitch
+    uint32_t L, Lp;     // product of the earlier radices; the same one stage before
+    uint32_t rstep;     // LDS step between a butterfly's points
+    uint32_t twoff;     // stage offset in the stage-twiddle table
+    uint32_t dnr, dL, dLp;
+};
+struct Mix {
+    uint32_t n, ns;
+    uint32_t lpw, nt;  // lines and threads of a workgroup
+    uint32_t lstr;     // LDS elements per line
+    uint32_t pp;       // offset of the second buffer; 0: one buffer
+    uint32_t ld_lf, st_lf, dlpw;
+    MixStage st[kMixStages];
+};
+std::vector<int> mix_schedule(uint64_t n);
+// Tile of `lines` lines of n points within `budget` bytes of LDS; fixed_nt /
+// forced_lpw pin the threads and lines of a workgroup (0: chosen).
+bool mix_plan(int arith, uint64_t n, uint64_t lines, bool ld_lf, bool st_lf, size_t budget, uint32_t fixed_nt,
+              uint32_t forced_lpw, Mix* out);
+size_t mix_lds_bytes(int arith, const Mix& x);
+hipError_t launch_mix_f32(int ldm, int stm, int post, const LineArgs& a, const Mix& mx, hipStream_t s);
+hipError_t launch_mix_f64(int ldm, int stm, int post, const LineArgs& a, const Mix& mx, hipStream_t s);
+hipError_t launch_mix_df64(int ldm, int stm, int post, const LineArgs& a, const Mix& mx, hipStream_t s);
+inline hipError_t launch_mix(int prec, int ldm, int stm, int post, const LineArgs& a, const Mix& mx, hipStream_t s) {
+    return prec == P_F32   ? launch_mix_f32(ldm, stm, post, a, mx, s)
+           : prec == P_F64 ? launch_mix_f64(ldm, stm, post, a, mx, s)
+                           : launch_mix_df64(ldm, stm, post, a, mx, s);
+}
+
 // Fused Rader / Bluestein convolution kernels (one line per workgroup pass).
 struct ConvArgs {
     LineArgs io;              // the prime / Bluestein line layout (n points)

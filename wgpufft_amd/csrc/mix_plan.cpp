@@ -1,0 +1,214 @@
+// Host side of the runtime-schedule register kernels (mix_kernels.hpp): the
+// radix schedule of a length and the shape (lines, threads, LDS) of a tile.
+#include <algorithm>
+#include <cmath>
+#include <cstring>
+#include <map>
+#include <mutex>
+
+#include "launch.h"
+
+namespace mifft {
+
+// Arithmetic instructions of a radix-R butterfly (fft_math.hpp: symmetric
+// pairs for odd primes, two factors for composites, without a twiddle between
+// coprime ones).
+static double butterfly_ops(int r) {
+    static const double ops[17] = {0, 0, 4, 14, 16, 36, 40, 66, 56, 100, 92, 150, 104, 204, 160, 178, 160};
+    return ops[r];
+}
+// Work of one stage per point: the butterfly, and in the same unit the
+// twiddle multiply, one LDS write and read with their addresses and a share
+// of the exchange's latency.
+static double stage_cost(int r) { return butterfly_ops(r) / r + 14.0; }
+
+static uint32_t mix_mag(uint32_t d) { return d <= 1 ? 0u : (uint32_t)(((1ull << 32) + d - 1) / d); }
+
+// Smallest compiled unroll (MIFFT_MIX_RADICES) that covers `need`
+// butterflies of radix r per thread, or the largest.
+static uint32_t nb_for(int r, uint32_t need) {
+    switch (r) {
+        case 2: case 3: return 4;
+        case 4: return need <= 1 ? 1 : 4;
+        case 5: return need <= 1 ? 1 : 3;
+        case 6: case 7: return 2;
+        case 8: return need <= 1 ? 1 : 2;
+        default: return 1;
+    }
+}
+
+static Mix shape(uint64_t n, const std::vector<int>& rad, uint32_t lpw, uint32_t nt, bool ld_lf, bool st_lf) {
+    Mix x;
+    std::memset(&x, 0, sizeof(x));
+    x.n = (uint32_t)n;
+    x.ns = (uint32_t)rad.size();
+    x.lpw = lpw;
+    x.nt = nt;
+    x.ld_lf = ld_lf;
+    x.st_lf = st_lf;
+    x.dlpw = mix_mag(lpw);
+    uint32_t L = 1, twoff = 0;
+    bool pp = false;
+    for (uint32_t s = 0; s < x.ns; s++) {
+        MixStage& st = x.st[s];
+        const uint32_t R = (uint32_t)rad[s], nr = (uint32_t)n / R;
+        const uint32_t need = (lpw * nr + nt - 1) / nt, nb = nb_for((int)R, need);
+        st.code = R + 32 * nb;
+        st.nr = nr;
+        st.nrp = nr | 1u;
+        st.L = L;
+        st.Lp = s ? L / (uint32_t)rad[s - 1] : 1;
+        st.nrp_prev = s ? x.st[s - 1].nrp : 0;
+        st.rstep = ((uint32_t)n / (L * R)) * st.Lp;
+        st.twoff = twoff;
+        st.dnr = mix_mag(nr);
+        st.dL = mix_mag(L);
+        st.dLp = mix_mag(st.Lp);
+        if (s >= 1) twoff += (R - 1) * L;
+        if (s + 1 < x.ns) x.lstr = std::max(x.lstr, R * st.nrp);
+        // a middle stage that takes more than one round writes a second buffer
+        if (s >= 1 && s + 1 < x.ns && need > nb) pp = true;
+        L *= R;
+    }
+    x.lstr |= 1u;
+    x.pp = pp ? lpw * x.lstr : 0;
+    return x;
+}
+
+size_t mix_lds_bytes(int arith, const Mix& x) {
+    if (x.ns <= 1) return 0;
+    return (size_t)(x.pp ? 2 : 1) * x.lpw * x.lstr * (arith == P_F32 ? 8 : 16);
+}
+
+// Relative rate of a tile shape, 1 at best.  Fitted to 8 Mi-point passes of
+// 15 lengths from 60 to 7680 points, f32 and f64, contiguous and strided,
+// over every thread count: the best contiguous shapes are one to a few lines
+// in 64 to 256 threads (1080 points: 1 line, 128 threads 28.5 us; 4 lines,
+// 512 threads 33.3 us; 576 threads 45 us), since a barrier then holds up few
+// waves; more than 256 threads cost 10 to 30 %, most where they are not a
+// multiple of the four SIMDs' waves.
+static double shape_score(int arith, const Mix& x, uint64_t lines, bool lf) {
+    const size_t es = arith == P_F32 ? 8 : 16, lds = mix_lds_bytes(arith, x);
+    // share of the launched lanes' butterfly slots that do work
+    double useful = 0, slots = 0;
+    for (uint32_t s = 0; s < x.ns; s++) {
+        const uint32_t R = x.st[s].code & 31u, nb = x.st[s].code >> 5, total = x.lpw * x.st[s].nr;
+        const double w = butterfly_ops((int)R) + 8.0 * R;
+        const uint32_t rounds = (total + x.nt * nb - 1) / (x.nt * nb);
+        useful += w * total;
+        slots += w * rounds * nb * x.nt;
+    }
+    double score = useful / slots;
+    score *= x.nt <= 256 ? 1.0 : x.nt < 512 ? 0.80 : x.nt == 512 ? 0.78 : 0.68;
+    // threads resident on a CU hide the barriers and the memory latency of one
+    // another (82 registers in f32, 128 to 158 in f64)
+    const double reg_threads = arith == P_F32 ? 1280 : 1024;
+    const double wgs_cu = std::floor(std::min((double)kLdsBudget / (double)lds, std::max(1.0, reg_threads / x.nt)));
+    score *= std::sqrt(std::min(1.0, wgs_cu * x.nt / 1024.0));
+    // strided sides: the row segment of a tile; neighbouring tiles run on the
+    // same XCD and share what is left of a line through its L2
+    if (lf) {
+        const size_t seg = x.lpw * es;
+        score *= seg >= 128 ? 1.0 : seg >= 64 ? 0.97 : seg >= 32 ? 0.9 : seg >= 16 ? 0.7 : 0.4;
+    }
+    // at least two workgroups per CU where the lines allow it
+    const double wgs = std::ceil((double)lines / x.lpw), want = 2.0 * device_cu_count();
+    if (wgs < want && x.lpw > 1) score *= 0.3 + 0.7 * wgs / want;
+    return score;
+}
+
+static double best_shape(int arith, uint64_t n, const std::vector<int>& rad, uint64_t lines, bool ld_lf, bool st_lf,
+                         size_t budget, uint32_t fixed_nt, uint32_t forced_lpw, bool pp, Mix* out) {
+    static const uint32_t threads[] = {64, 128, 192, 256, 320, 384, 448, 512, 640, 768, 1024};
+    const bool lf = ld_lf || st_lf;
+    double best = -1;
+    for (uint32_t nt : threads) {
+        if (fixed_nt && nt != fixed_nt) continue;
+        for (uint32_t lpw = forced_lpw ? forced_lpw : 1; lpw <= (forced_lpw ? forced_lpw : 64); lpw = lf && !forced_lpw ? 2 * lpw : lpw + 1) {
+            if ((lpw > lines && lpw > 1 && !forced_lpw) || (uint64_t)lpw * n > 0xFFFFu) break;
+            // (more than two rounds of 16 points per thread, or under two
+            // points: never the best shape)
+            if (!fixed_nt && !forced_lpw && lpw > 1 && (uint64_t)lpw * n > 34ull * nt) break;
+            if (!fixed_nt && !forced_lpw && nt > 64 && (uint64_t)lpw * n < 2ull * nt) continue;
+            const Mix x = shape(n, rad, lpw, nt, ld_lf, st_lf);
+            if (mix_lds_bytes(arith, x) > budget || (x.pp && !pp)) break;
+            const double score = shape_score(arith, x, lines, lf);
+            if (score > best + 1e-9) {
+                best = score;
+                if (out) *out = x;
+            }
+        }
+    }
+    return best;
+}
+
+static void multisets(uint64_t n, int max_r, double cost, std::vector<int>& cur, double& best,
+                      std::vector<std::pair<double, std::vector<int>>>& out) {
+    if (n == 1) {
+        best = std::min(best, cost);
+        out.emplace_back(cost, cur);
+        return;
+    }
+    if (cur.size() >= (size_t)kMixStages) return;
+    for (int r = max_r; r >= 2; r--) {
+        if (n % (uint64_t)r) continue;
+        const double c = cost + stage_cost(r);
+        if (c > 1.3 * best) continue;
+        cur.push_back(r);
+        multisets(n / (uint64_t)r, r, c, cur, best, out);
+        cur.pop_back();
+    }
+}
+
+// The schedule of n: over the radix multisets within 30 % of the cheapest and
+// their orders, the least work per point over the rate of its best contiguous
+// tile (the fill of the threads decides between, for 1080 points, 15x9x8 at
+// 45 us and 12x10x9 at 28 us per 8 Mi points).  The larger radix first where
+// nothing else decides (12x9 23.9 us, 9x12 25.7 us).  It depends on n alone:
+// a line's result does not depend on the tile, the precision of its
+// neighbours or their number.
+std::vector<int> mix_schedule(uint64_t n) {
+    static std::mutex mu;
+    static std::map<uint64_t, std::vector<int>> done;  // at most the smooth lengths up to 2^15
+    if (n < 2 || n > 0x8000u) return {};
+    std::lock_guard<std::mutex> g(mu);
+    auto f = done.find(n);
+    if (f != done.end()) return f->second;
+    std::vector<std::pair<double, std::vector<int>>> sets;
+    std::vector<int> cur, best;
+    double least = 1e30;
+    multisets(n, 16, 0, cur, least, sets);
+    double value = 1e30;
+    for (auto& s : sets) {
+        if (s.first > 1.3 * least) continue;
+        std::vector<int> r = s.second;
+        std::sort(r.begin(), r.end());
+        do {
+            double score = r.size() < 2 ? 1.0
+                                        : best_shape(P_F32, n, r, 1u << 30, false, false, kLdsBudget, 0, 0, false, nullptr);
+            if (score <= 0) score = 1e-3;
+            const double v = s.first / score * (r.front() < r.back() ? 1.02 : 1.0) * (r.front() < r[r.size() > 1] ? 1.01 : 1.0);
+            if (v < value) {
+                value = v;
+                best = r;
+            }
+        } while (std::next_permutation(r.begin(), r.end()));
+    }
+    done[n] = best;
+    return best;
+}
+
+bool mix_plan(int arith, uint64_t n, uint64_t lines, bool ld_lf, bool st_lf, size_t budget, uint32_t fixed_nt,
+              uint32_t forced_lpw, Mix* out) {
+    const std::vector<int> rad = mix_schedule(n);
+    if (rad.size() < 2 || !lines) return false;
+    // batched tiles: the launch's LDS is its largest tile's, so half the
+    // budget (four workgroups per CU) where the line fits it; a second buffer
+    // (several rounds per middle stage) only where nothing else does
+    for (int pp = 0; pp < 2; pp++)
+        for (size_t b : {fixed_nt ? budget / 2 : budget, budget})
+            if (best_shape(arith, n, rad, lines, ld_lf, st_lf, b, fixed_nt, forced_lpw, pp, out) > 0) return true;
+    return false;
+}
+
+}  // namespace mifft

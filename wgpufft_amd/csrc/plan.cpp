@@ -422,6 +422,12 @@ static Sched make_sched(uint64_t n, uint32_t lpw, bool ld_lf, bool st_lf, const 
     return sc;
 }
 
+static std::string radices_str(const std::vector<int>& rad) {
+    std::string s;
+    for (size_t i = 0; i < rad.size(); i++) s += (i ? "x" : "") + std::to_string(rad[i]);
+    return s;
+}
+
 static std::string sched_str(const Sched& sc) {
     std::string s;
     for (uint32_t i = 0; i < sc.ns; i++) s += (i ? "x" : "") + std::to_string(sc.rad[i]);
@@ -629,6 +635,39 @@ struct Builder {
         return best;
     }
 
+    // Makes `op` (lines, lane layout and modes set) a runtime-schedule line
+    // op: the register form (mix_kernels.hpp) for complex lines of at least two
+    // stages, else the LDS-to-LDS one.  The radix schedule depends on the
+    // length alone, so a line's result does not depend on its neighbours or on
+    // the tile.
+    void runtime_schedule(Op& op, bool batched, uint32_t forced_lpw) {
+        op.kind = OP_LDS;
+        op.rv = nullptr;
+        op.mix = Mix{};
+        const uint64_t n = op.n;
+        const size_t es = elem_bytes(P.arith);
+        const uint32_t fit = (uint32_t)(P.lds_budget / (2 * lds_line_stride((uint32_t)n) * es));
+        if (op.ldm == LD_COMPLEX && op.stm == ST_COMPLEX) {
+            bool ok = false;
+            for (uint32_t lpw = forced_lpw; !ok; lpw--) {
+                ok = mix_plan(P.arith, n, op.a.lines, op.ld_lf, op.st_lf, P.lds_budget, batched ? 256 : 0, lpw, &op.mix);
+                if (lpw <= 1) break;
+            }
+            if (ok) {
+                op.a.tw = stage_twiddles(P.arith, mix_schedule(n));
+                return;
+            }
+            op.mix = Mix{};
+        }
+        uint32_t lpw;
+        if (op.ld_lf || op.st_lf) lpw = P.arith == P_F32 ? 16 : 8;
+        else lpw = (uint32_t)std::max<uint64_t>(1, 4096 / n);
+        if (forced_lpw) lpw = forced_lpw;
+        lpw = std::max<uint32_t>(1, std::min(lpw, fit));
+        op.sc = make_sched(n, lpw, op.ld_lf, op.st_lf);
+        op.a.tw = stage_twiddles(P.arith, sched_radices(op.sc));
+    }
+
     // One line kernel (register variant when compiled, else the LDS kernel).
     // Returns false if the line does not fit on chip.
     bool line_op(uint64_t n, const LineSet& ls, const Layout& in, const Layout& out, int src,
@@ -721,16 +760,10 @@ struct Builder {
               << " lpw=" << rv->lines;
             if (rv->persist) d << " pipe" << rv->persist;
         } else {
-            op.kind = OP_LDS;
-            uint32_t fit = (uint32_t)(P.lds_budget / (2 * lstr * es));
-            uint32_t lpw;
-            if (ld_lf || st_lf) lpw = P.arith == P_F32 ? 16 : 8;
-            else lpw = (uint32_t)std::max<uint64_t>(1, 4096 / n);
-            if (forced_lpw) lpw = forced_lpw;
-            lpw = std::max<uint32_t>(1, std::min(lpw, fit));
-            op.sc = make_sched(n, lpw, ld_lf, st_lf);
-            op.a.tw = stage_twiddles(P.arith, sched_radices(op.sc));
-            d << "lds N=" << n << " " << sched_str(op.sc) << " lines=" << ls.lines << " lpw=" << lpw;
+            runtime_schedule(op, P.batch_mode, forced_lpw);
+            d << "lds N=" << n << " " << (op.mix.ns ? radices_str(mix_schedule(n)) : sched_str(op.sc))
+              << " lines=" << ls.lines << " lpw=" << (op.mix.ns ? op.mix.lpw : op.sc.lpw);
+            if (op.mix.ns) d << " nt=" << op.mix.nt << (op.mix.pp ? " pp" : "");
         }
         if (ld_lf || st_lf) d << (ld_lf ? " ldLF" : "") << (st_lf ? " stLF" : "");
         if (post) d << " post";
@@ -1874,7 +1907,9 @@ static void run_op(const Op& op, hipStream_t s, const void* in, void* out, void*
             LineArgs a = op.a;
             a.in = ptr(op.src, op.src_off);
             a.out = ptr(op.dst, op.dst_off);
-            hip_check(launch_lds(op.prec, op.ldm, op.stm, op.post, a, op.sc, s), "LDS line kernel");
+            hip_check(op.mix.ns ? launch_mix(op.prec, op.ldm, op.stm, op.post, a, op.mix, s)
+                                : launch_lds(op.prec, op.ldm, op.stm, op.post, a, op.sc, s),
+                      "LDS line kernel");
             break;
         }
         case OP_RADER:
@@ -2233,10 +2268,7 @@ int autotune_sequence(const mifft_config* cfgs, const mifft_kind* kinds, int cou
             for (uint32_t lpw = 1; lpw <= 32 && !ref->fold; lpw *= 2) {
                 if (2 * lstr * es * lpw > T.lds_budget || lpw > ref->a.lines) break;
                 Op c = *ref;
-                c.kind = OP_LDS;
-                c.rv = nullptr;
-                c.sc = make_sched(ref->n, lpw, ref->ld_lf, ref->st_lf);
-                c.a.tw = TB.stage_twiddles(ref->prec == P_F32 ? P_F32 : P_F64, Builder::sched_radices(c.sc));
+                TB.runtime_schedule(c, false, lpw);
                 cands.emplace_back("lds:lpw=" + std::to_string(lpw), c);
             }
             if (cands.size() < 2) continue;
@@ -2248,6 +2280,7 @@ int autotune_sequence(const mifft_config* cfgs, const mifft_kind* kinds, int cou
                             o.kind = c.kind;
                             o.rv = c.rv;
                             o.sc = c.sc;
+                            o.mix = c.mix;
                             o.a.tw = c.a.tw;
                         }
             };

@@ -53,6 +53,7 @@ struct Op {
     int prec = P_F32;                   // kernel format
     LineArgs a{};
     Sched sc{};
+    Mix mix{};          // OP_LDS: the register form's tile (ns > 0), instead of sc
     ConvArgs conv{};
     SmallVolArgs sv{};  // OP_SMALL_VOLUME (volumes in count)
     StockhamStage st{}; // OP_STOCKHAM
