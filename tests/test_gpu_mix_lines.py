@@ -92,3 +92,33 @@ def test_batched_tiles_equal_standalone(torch_cuda):
     for it, w in zip(items, want):
         got = from_dev(it["output"], np.complex64)
         assert np.array_equal(got.view(np.uint32), w.view(np.uint32)), it["n"]
+
+
+@pytest.mark.parametrize("n", [36, 60, 66, 98, 120, 286, 400, 1014, 1920, 4374, 9000])
+@pytest.mark.parametrize("batch", [1, 13])
+def test_half_length_real_lines(torch_cuda, n, batch):
+    """Even real lines at half length; C2R drops the imaginary parts of the
+    first and last bin of arbitrary packed input, as numpy's irfft does."""
+    rng = np.random.default_rng(n + batch)
+    x = rng.uniform(-1, 1, (batch, n)).astype(np.float32)
+    r2c = FftPlan.r2c(FftConfig.new(n).with_batch(batch))
+    assert "half" in r2c.describe(), r2c.describe()
+    y = run(r2c, x, batch * (n // 2 + 1) * 8).view(np.complex64)
+    e = oracle.rel_l2(y, np.fft.rfft(x.astype(np.float64), axis=1).reshape(-1))
+    assert e <= 1e-6, (n, batch, e, r2c.describe())
+    p = seeded_complex(n, batch * (n // 2 + 1))
+    c2r = FftPlan.c2r(FftConfig.inverse(n).with_batch(batch))
+    assert "half" in c2r.describe(), c2r.describe()
+    z = run(c2r, p, batch * n * 4).view(np.float32)
+    e = oracle.rel_l2(z, np.fft.irfft(p.astype(np.complex128).reshape(batch, -1), n=n, axis=1).reshape(-1))
+    assert e <= 1e-6, (n, batch, e, c2r.describe())
+
+
+def test_half_length_real_volume(torch_cuda):
+    shape, batch = [60, 18, 35], 2
+    x = np.random.default_rng(3).uniform(-1, 1, (batch, 35, 18, 60)).astype(np.float32)
+    r2c, c2r = FftPlan.r2c(FftConfig.new_nd(shape).with_batch(batch)), FftPlan.c2r(FftConfig.inverse_nd(shape).with_batch(batch))
+    y = run(r2c, x, batch * 35 * 18 * 31 * 8).view(np.complex64)
+    assert oracle.rel_l2(y, np.fft.rfftn(x.astype(np.float64), axes=(1, 2, 3)).reshape(-1)) <= 1e-6
+    z = run(c2r, y, x.nbytes).view(np.float32)
+    assert oracle.rel_l2(z, x.astype(np.float64).reshape(-1)) <= 1e-6

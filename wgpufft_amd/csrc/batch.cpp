@@ -219,8 +219,8 @@ void batch_build(const BatchEntry* entries, int32_t count, char* ws_base, BatchB
                     // a plan made for one line: the tile for all lines that run it
                     if (op.mix.ns && e.mult > 1) {
                         Mix m;
-                        if (mix_plan(P.arith, op.n, (uint64_t)op.a.lines * e.mult, op.ld_lf, op.st_lf, P.lds_budget, 256,
-                                     0, &m))
+                        if (mix_plan(P.arith, op.mix.n, (uint64_t)op.a.lines * e.mult, op.ld_lf, op.st_lf, P.lds_budget,
+                                     256, 0, op.mix.pairs > 0, &m))
                             d.mix = m;
                     }
                     lpw = d.mix.ns ? d.mix.lpw : op.sc.lpw;

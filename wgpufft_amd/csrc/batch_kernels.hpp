@@ -65,6 +65,8 @@ enum BatchClass : uint32_t {
     BC_MIX_POST,
     BC_MIX_F64,
     BC_MIX_POST_F64,
+    BC_MIX_R2C,  // even real lines at half length
+    BC_MIX_C2R,
     BC_COUNT
 };
 
@@ -85,8 +87,8 @@ struct BatchTile {
 // Arguments of one op of one transform, device pointers already bound.
 struct OpDesc {
     LineArgs a;   // line ops (register and LDS classes)
-    Sched sc;     // LDS classes of real lines
-    Mix mix;      // LDS classes of complex lines
+    Sched sc;     // LDS-to-LDS classes
+    Mix mix;      // BC_MIX classes
     ConvArgs conv;  // Rader / Bluestein classes; element-wise classes (io, chirp, filt, n, m)
 };
 

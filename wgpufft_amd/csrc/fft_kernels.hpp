@@ -45,6 +45,8 @@ struct LineArgs {
     // Fold passes (F lines per thread): line c of a fold group sits c times
     // these element offsets after the first, which is at line_base(g / F).
     uint32_t fold_in, fold_out;
+    // Half-length real lines (mix_real_tile): W_{2n}^k for k <= n / 2.
+    const void* half_tw;
 };
 
 __device__ __forceinline__ uint32_t xcd_remap(uint32_t b, uint32_t n) {

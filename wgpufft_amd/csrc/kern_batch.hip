@@ -91,6 +91,11 @@ __device__ __noinline__ uint32_t mix_tiles(MIFFT_TILE_ARGS) {
         mix_tile<Fmt, LD_COMPLEX, ST_COMPLEX, POST>(d.a, d.mix, smem, g0);
     });
 }
+template <bool C2R>
+__device__ __noinline__ uint32_t mix_real_tiles(MIFFT_TILE_ARGS) {
+    return tile_run(tiles, ntiles, counter, ops, t,
+                    [&](const OpDesc& d, uint32_t g0) { mix_real_tile<C2R>(d.a, d.mix, smem, g0); });
+}
 template <class Fmt, bool MED = false>
 __device__ __noinline__ uint32_t rader_tiles(MIFFT_TILE_ARGS) {
     return tile_run(tiles, ntiles, counter, ops, t,
@@ -151,6 +156,8 @@ __global__ void __launch_bounds__(256, 4) k_batch(const BatchTile* __restrict__ 
             case BC_MIX_POST: t = mix_tiles<FmtF32, true>(MIFFT_TILE_PASS); break;
             case BC_MIX_F64: t = mix_tiles<FmtF64, false>(MIFFT_TILE_PASS); break;
             case BC_MIX_POST_F64: t = mix_tiles<FmtF64, true>(MIFFT_TILE_PASS); break;
+            case BC_MIX_R2C: t = mix_real_tiles<false>(MIFFT_TILE_PASS); break;
+            case BC_MIX_C2R: t = mix_real_tiles<true>(MIFFT_TILE_PASS); break;
             case BC_RADER: t = rader_tiles<FmtF32>(MIFFT_TILE_PASS); break;
             case BC_BLUESTEIN: t = bluestein_tiles<FmtF32>(MIFFT_TILE_PASS); break;
             case BC_RADER_F64: t = rader_tiles<FmtF64>(MIFFT_TILE_PASS); break;
@@ -227,8 +234,8 @@ int batch_lds_class(int prec, int ldm, int stm, int post, bool mix) {
         if (prec == P_F64) return mix ? (post ? BC_MIX_POST_F64 : BC_MIX_F64) : (post ? BC_LDS_POST_F64 : BC_LDS_F64);
         return -1;
     }
-    if (prec == P_F32 && !post && ldm == LD_REAL && stm == ST_PACKED) return BC_LDS_R2C;
-    if (prec == P_F32 && !post && ldm == LD_HERMITIAN && stm == ST_REAL) return BC_LDS_C2R;
+    if (prec == P_F32 && !post && ldm == LD_REAL && stm == ST_PACKED) return mix ? BC_MIX_R2C : BC_LDS_R2C;
+    if (prec == P_F32 && !post && ldm == LD_HERMITIAN && stm == ST_REAL) return mix ? BC_MIX_C2R : BC_LDS_C2R;
     return -1;
 }
 

@@ -424,14 +424,15 @@ static hipError_t launch_lds_fmt(int ldm, int stm, int post, const LineArgs& a, 
     else if (ldm == LD_COMPLEX && stm == ST_COMPLEX && post)
         fn = wide ? (const void*)&lds_fft_kernel<Fmt, LD_COMPLEX, ST_COMPLEX, true, 512>
                   : (const void*)&lds_fft_kernel<Fmt, LD_COMPLEX, ST_COMPLEX, true>;
-    else if (ldm == LD_REAL && stm == ST_PACKED && !post)
-        fn = wide ? (const void*)&lds_fft_kernel<Fmt, LD_REAL, ST_PACKED, false, 512>
-                  : (const void*)&lds_fft_kernel<Fmt, LD_REAL, ST_PACKED, false>;
-    else if (ldm == LD_HERMITIAN && stm == ST_REAL && !post)
-        fn = wide ? (const void*)&lds_fft_kernel<Fmt, LD_HERMITIAN, ST_REAL, false, 512>
-                  : (const void*)&lds_fft_kernel<Fmt, LD_HERMITIAN, ST_REAL, false>;
-    else
-        return hipErrorInvalidValue;
+    else if constexpr (Fmt::kId == 0) {  // real lines (odd, or up to 32 points): f32 only
+        if (ldm == LD_REAL && stm == ST_PACKED && !post)
+            fn = wide ? (const void*)&lds_fft_kernel<Fmt, LD_REAL, ST_PACKED, false, 512>
+                      : (const void*)&lds_fft_kernel<Fmt, LD_REAL, ST_PACKED, false>;
+        else if (ldm == LD_HERMITIAN && stm == ST_REAL && !post)
+            fn = wide ? (const void*)&lds_fft_kernel<Fmt, LD_HERMITIAN, ST_REAL, false, 512>
+                      : (const void*)&lds_fft_kernel<Fmt, LD_HERMITIAN, ST_REAL, false>;
+    }
+    if (!fn) return hipErrorInvalidValue;
     hipError_t e = ensure_lds_attr(fn, bytes);
     if (e != hipSuccess) return e;
     const uint32_t blocks = (a.lines + sc.lpw - 1) / sc.lpw;

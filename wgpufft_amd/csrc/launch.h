@@ -84,18 +84,24 @@ struct Mix {
     uint32_t lstr;     // LDS elements per line
     uint32_t pp;       // offset of the second buffer; 0: one buffer
     uint32_t ld_lf, st_lf, dlpw;
+    // half-length real lines (n complex points of 2n real ones): bin pairs
+    // k, n - k per line, n / 2 + 1 of them; 0 for complex lines
+    uint32_t pairs, dpairs;
     MixStage st[kMixStages];
 };
 std::vector<int> mix_schedule(uint64_t n);
 // Tile of `lines` lines of n points within `budget` bytes of LDS; fixed_nt /
 // forced_lpw pin the threads and lines of a workgroup (0: chosen).
+// `real`: lines of 2n real points at half length.
 bool mix_plan(int arith, uint64_t n, uint64_t lines, bool ld_lf, bool st_lf, size_t budget, uint32_t fixed_nt,
-              uint32_t forced_lpw, Mix* out);
+              uint32_t forced_lpw, bool real, Mix* out);
 size_t mix_lds_bytes(int arith, const Mix& x);
 hipError_t launch_mix_f32(int ldm, int stm, int post, const LineArgs& a, const Mix& mx, hipStream_t s);
 hipError_t launch_mix_f64(int ldm, int stm, int post, const LineArgs& a, const Mix& mx, hipStream_t s);
 hipError_t launch_mix_df64(int ldm, int stm, int post, const LineArgs& a, const Mix& mx, hipStream_t s);
+hipError_t launch_mix_real(bool c2r, const LineArgs& a, const Mix& mx, hipStream_t s);
 inline hipError_t launch_mix(int prec, int ldm, int stm, int post, const LineArgs& a, const Mix& mx, hipStream_t s) {
+    if (mx.pairs) return launch_mix_real(ldm == LD_HERMITIAN, a, mx, s);
     return prec == P_F32   ? launch_mix_f32(ldm, stm, post, a, mx, s)
            : prec == P_F64 ? launch_mix_f64(ldm, stm, post, a, mx, s)
                            : launch_mix_df64(ldm, stm, post, a, mx, s);

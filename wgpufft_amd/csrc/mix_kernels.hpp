@@ -219,6 +219,189 @@ __device__ __forceinline__ void mix_tile(const LineArgs& a, const Mix& mx, unsig
     }
 }
 
+// ------------------------------------------------ half-length real lines
+// A real line of N0 = 2n points read as n complex ones, z[m] = x[2m] + i
+// x[2m+1], with Z = DFT_n(z), has the bins (k <= n, W = W_N0^k)
+//   X[k] = A + W B,  X[n - k] = conj(A - W B),
+//   A = (Z[k] + conj Z[n-k]) / 2,  B = (Z[k] - conj Z[n-k]) / 2i;
+// the inverse starts from
+//   Z[k] = E + i O,  Z[n-k] = conj E + i conj O,
+//   E = X[k] + conj X[n-k],  O = (X[k] - conj X[n-k]) conj W
+// (the imaginary parts of bins 0 and n are dropped).  Half the points go
+// through the stages, and the pairs k, n - k meet in LDS in natural order:
+// one exchange more than a complex line of n points, where the full-length
+// form runs N0-point lines whose upper half it drops.  48000 x 400 R2C 118 ->
+// 44 us (154 MB, 3.5 TB/s; 30 us at the copy rate), 1920x1080x3 R2C + C2R 127
+// -> 75 us, 144x120x108 52 -> 44 us.
+
+// A stage from LDS to LDS whose side NAT_IN reads / NAT_OUT writes natural
+// point order (stage 0 after, the last stage before the bin pairs); as mix_mid
+// otherwise.
+template <int R, int NB, bool NAT_IN, class T>
+__device__ __forceinline__ void mix_nat(const Mix& mx, const MixStage& st, const cpx<T>* src, cpx<T>* dst, const void* tw) {
+    const uint32_t total = mx.lpw * st.nr;
+    for (uint32_t r0 = 0; r0 < total; r0 += blockDim.x * NB) {
+        const uint32_t b0 = r0 + threadIdx.x;
+        cpx<T> w[NB][R];
+        MixPos at[NB];
+#pragma unroll
+        for (int q = 0; q < NB; q++) {
+            const uint32_t b = b0 + q * blockDim.x;
+            at[q] = mix_pos(mx, st, b < total ? b : total - 1, false);
+        }
+        if constexpr (NAT_IN) {
+#pragma unroll
+            for (int q = 0; q < NB; q++)
+#pragma unroll
+                for (int i = 0; i < R; i++) w[q][i] = src[at[q].lg * mx.lstr + at[q].j + i * st.nr];
+#pragma unroll
+            for (int q = 0; q < NB; q++) Dft<R, T>::run(w[q]);
+        } else {
+            mix_take<R, NB, T>(mx, st, src, tw, at, w);
+        }
+        if (!mx.pp) __syncthreads();
+#pragma unroll
+        for (int q = 0; q < NB; q++)
+            if (b0 + q * blockDim.x < total) {
+                if constexpr (NAT_IN) {
+                    mix_put<R, T>(mx, st, dst, at[q], w[q]);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < R; i++) dst[at[q].lg * mx.lstr + at[q].j + i * st.nr] = w[q][i];
+                }
+            }
+    }
+}
+
+// Bin pairs in flight per thread.
+constexpr uint32_t kMixPairs = 4;
+
+// R2C: LDS (natural order) -> packed bins.
+template <class T>
+__device__ __forceinline__ void mix_pairs_out(const LineArgs& a, const Mix& mx, const cpx<T>* z, uint32_t g0) {
+    const uint32_t n = mx.n, total = mx.lpw * mx.pairs;
+    const T sc = T(0.5) * (T)a.scale;  // the halves of A and B (exact)
+    for (uint32_t t0 = threadIdx.x; t0 < total; t0 += blockDim.x) {
+        const uint32_t lg = mix_div(t0, mx.dpairs), k = t0 - lg * mx.pairs, g = g0 + lg;
+        if (g >= a.lines) return;
+        const cpx<T> w = ld_tw<T>(a.half_tw, k);
+        const cpx<T>* zl = z + lg * mx.lstr;
+        const cpx<T> p = zl[k], q = zl[k ? n - k : 0];
+        const cpx<T> A = mk<T>(p.x + q.x, p.y - q.y), B = mk<T>(p.y + q.y, q.x - p.x);
+        // A +- W B with two roundings per component
+        const cpx<T> u = mk<T>(fma(-w.y, B.y, fma(w.x, B.x, A.x)), fma(w.y, B.x, fma(w.x, B.y, A.y)));
+        const cpx<T> v = mk<T>(fma(w.y, B.y, fma(-w.x, B.x, A.x)), fma(-w.y, B.x, fma(-w.x, B.y, A.y)));
+        const uint32_t o = line_base(a, g).out;
+        FmtF32::st(a.out, o + k, mk<T>(u.x * sc, u.y * sc));
+        if (2 * k != n) FmtF32::st(a.out, o + n - k, mk<T>(v.x * sc, -v.y * sc));
+    }
+}
+
+// C2R: packed bins -> LDS, conjugated (the inverse is conj DFT conj).
+template <class T>
+__device__ __forceinline__ void mix_pairs_in(const LineArgs& a, const Mix& mx, cpx<T>* z, uint32_t g0) {
+    const uint32_t n = mx.n, total = mx.lpw * mx.pairs;
+    for (uint32_t t0 = threadIdx.x; t0 < total; t0 += blockDim.x * kMixPairs) {
+        cpx<T> p[kMixPairs], q[kMixPairs], w[kMixPairs];
+        uint32_t lg[kMixPairs], k[kMixPairs];
+#pragma unroll
+        for (uint32_t u = 0; u < kMixPairs; u++) {
+            const uint32_t t = t0 + u * blockDim.x, tc = t < total ? t : total - 1;
+            lg[u] = mix_div(tc, mx.dpairs);
+            k[u] = tc - lg[u] * mx.pairs;
+            const uint32_t g = g0 + lg[u], o = line_base(a, g < a.lines ? g : a.lines - 1).in;
+            p[u] = FmtF32::ld_c(a.in, o + k[u]);
+            q[u] = FmtF32::ld_c(a.in, o + n - k[u]);
+            w[u] = ld_tw<T>(a.half_tw, k[u]);
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < kMixPairs; u++) {
+            if (t0 + u * blockDim.x >= total) break;
+            if (k[u] == 0) p[u].y = q[u].y = T(0);
+            const cpx<T> E = mk<T>(p[u].x + q[u].x, p[u].y - q[u].y), D = mk<T>(p[u].x - q[u].x, p[u].y + q[u].y);
+            const T wx = w[u].x, wy = w[u].y;
+            // E + i O and conj E + i conj O with O = D conj W, conjugated
+            cpx<T>* zl = z + lg[u] * mx.lstr;
+            zl[k[u]] = mk<T>(fma(wy, D.x, fma(-wx, D.y, E.x)), -fma(wy, D.y, fma(wx, D.x, E.y)));
+            if (k[u] && 2 * k[u] != n)
+                zl[n - k[u]] = mk<T>(fma(-wy, D.x, fma(wx, D.y, E.x)), fma(-wy, D.y, fma(-wx, D.x, E.y)));
+        }
+    }
+}
+
+// Lines [g0, g0 + lpw) of 2n real points (a's real side in complex elements).
+template <bool C2R>
+__device__ __forceinline__ void mix_real_tile(const LineArgs& a, const Mix& mx, unsigned char* smem, uint32_t g0) {
+    using T = float;
+    cpx<T>* src = reinterpret_cast<cpx<T>*>(smem);
+    cpx<T>* dst = src + mx.pp;
+    if constexpr (C2R) {
+        mix_pairs_in<T>(a, mx, src, g0);
+        __syncthreads();
+        const MixStage st = mx.st[0];
+        switch (st.code) {
+#define MIFFT_MIX_CASE(R, NB) \
+    case R + 32 * NB: mix_nat<R, NB, true, T>(mx, st, src, dst, a.tw); break;
+            MIFFT_MIX_RADICES(MIFFT_MIX_CASE)
+#undef MIFFT_MIX_CASE
+            default: break;
+        }
+        cpx<T>* x = src;
+        src = dst;
+        dst = x;
+    } else {
+        switch (mx.st[0].code) {
+#define MIFFT_MIX_CASE(R, NB) \
+    case R + 32 * NB: mix_first<FmtF32, LD_COMPLEX, R, NB>(a, mx, src, g0); break;
+            MIFFT_MIX_RADICES(MIFFT_MIX_CASE)
+#undef MIFFT_MIX_CASE
+            default: break;
+        }
+    }
+    __syncthreads();
+#pragma nounroll
+    for (uint32_t s = 1; s + 1 < mx.ns; s++) {
+        const MixStage st = mx.st[s];
+        switch (st.code) {
+#define MIFFT_MIX_CASE(R, NB) \
+    case R + 32 * NB: mix_mid<R, NB, T>(mx, st, src, dst, a.tw); break;
+            MIFFT_MIX_RADICES(MIFFT_MIX_CASE)
+#undef MIFFT_MIX_CASE
+            default: break;
+        }
+        __syncthreads();
+        cpx<T>* x = src;
+        src = dst;
+        dst = x;
+    }
+    const MixStage st = mx.st[mx.ns - 1];
+    if constexpr (C2R) {
+        switch (st.code) {
+#define MIFFT_MIX_CASE(R, NB) \
+    case R + 32 * NB: mix_last<FmtF32, ST_COMPLEX, false, R, NB>(a, mx, st, src, g0); break;
+            MIFFT_MIX_RADICES(MIFFT_MIX_CASE)
+#undef MIFFT_MIX_CASE
+            default: break;
+        }
+    } else {
+        switch (st.code) {
+#define MIFFT_MIX_CASE(R, NB) \
+    case R + 32 * NB: mix_nat<R, NB, false, T>(mx, st, src, dst, a.tw); break;
+            MIFFT_MIX_RADICES(MIFFT_MIX_CASE)
+#undef MIFFT_MIX_CASE
+            default: break;
+        }
+        __syncthreads();
+        mix_pairs_out<T>(a, mx, dst, g0);
+    }
+}
+
+template <bool C2R>
+__global__ void __launch_bounds__(1024) mix_real_kernel(LineArgs a, Mix mx) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    mix_real_tile<C2R>(a, mx, smem_raw, xcd_remap(blockIdx.x, gridDim.x) * mx.lpw);
+}
+
 // NT: the launch bound (the register budget).
 template <class Fmt, int LDM, int STM, bool POST, int NT>
 __global__ void __launch_bounds__(NT) mix_fft_kernel(LineArgs a, Mix mx) {

@@ -37,7 +37,8 @@ static uint32_t nb_for(int r, uint32_t need) {
     }
 }
 
-static Mix shape(uint64_t n, const std::vector<int>& rad, uint32_t lpw, uint32_t nt, bool ld_lf, bool st_lf) {
+static Mix shape(uint64_t n, const std::vector<int>& rad, uint32_t lpw, uint32_t nt, bool ld_lf, bool st_lf,
+                 bool real) {
     Mix x;
     std::memset(&x, 0, sizeof(x));
     x.n = (uint32_t)n;
@@ -47,6 +48,10 @@ static Mix shape(uint64_t n, const std::vector<int>& rad, uint32_t lpw, uint32_t
     x.ld_lf = ld_lf;
     x.st_lf = st_lf;
     x.dlpw = mix_mag(lpw);
+    if (real) {
+        x.pairs = x.n / 2 + 1;
+        x.dpairs = mix_mag(x.pairs);
+    }
     uint32_t L = 1, twoff = 0;
     bool pp = false;
     for (uint32_t s = 0; s < x.ns; s++) {
@@ -66,8 +71,10 @@ static Mix shape(uint64_t n, const std::vector<int>& rad, uint32_t lpw, uint32_t
         st.dLp = mix_mag(st.Lp);
         if (s >= 1) twoff += (R - 1) * L;
         if (s + 1 < x.ns) x.lstr = std::max(x.lstr, R * st.nrp);
-        // a middle stage that takes more than one round writes a second buffer
-        if (s >= 1 && s + 1 < x.ns && need > nb) pp = true;
+        // a stage from LDS to LDS that takes more than one round writes a
+        // second buffer: the middle stages, and the last (first) one where the
+        // bin pairs of real lines follow (precede) it
+        if ((real || (s >= 1 && s + 1 < x.ns)) && need > nb) pp = true;
         L *= R;
     }
     x.lstr |= 1u;
@@ -118,7 +125,7 @@ static double shape_score(int arith, const Mix& x, uint64_t lines, bool lf) {
 }
 
 static double best_shape(int arith, uint64_t n, const std::vector<int>& rad, uint64_t lines, bool ld_lf, bool st_lf,
-                         size_t budget, uint32_t fixed_nt, uint32_t forced_lpw, bool pp, Mix* out) {
+                         size_t budget, uint32_t fixed_nt, uint32_t forced_lpw, bool pp, bool real, Mix* out) {
     static const uint32_t threads[] = {64, 128, 192, 256, 320, 384, 448, 512, 640, 768, 1024};
     const bool lf = ld_lf || st_lf;
     double best = -1;
@@ -130,7 +137,7 @@ static double best_shape(int arith, uint64_t n, const std::vector<int>& rad, uin
             // points: never the best shape)
             if (!fixed_nt && !forced_lpw && lpw > 1 && (uint64_t)lpw * n > 34ull * nt) break;
             if (!fixed_nt && !forced_lpw && nt > 64 && (uint64_t)lpw * n < 2ull * nt) continue;
-            const Mix x = shape(n, rad, lpw, nt, ld_lf, st_lf);
+            const Mix x = shape(n, rad, lpw, nt, ld_lf, st_lf, real);
             if (mix_lds_bytes(arith, x) > budget || (x.pp && !pp)) break;
             const double score = shape_score(arith, x, lines, lf);
             if (score > best + 1e-9) {
@@ -164,9 +171,10 @@ static void multisets(uint64_t n, int max_r, double cost, std::vector<int>& cur,
 // their orders, the least work per point over the rate of its best contiguous
 // tile (the fill of the threads decides between, for 1080 points, 15x9x8 at
 // 45 us and 12x10x9 at 28 us per 8 Mi points).  The larger radix first where
-// nothing else decides (12x9 23.9 us, 9x12 25.7 us).  It depends on n alone:
-// a line's result does not depend on the tile, the precision of its
-// neighbours or their number.
+// nothing else decides (12x9 23.9 us, 9x12 25.7 us).  It depends on
+// the length alone: a line's result does not depend on the tile or on the
+// number of lines.  (Radices 18 and 20 measured: 270 points 36 -> 33 us, 1000
+// points 36 -> 38, 960-point half lines 4 % slower; not used.)
 std::vector<int> mix_schedule(uint64_t n) {
     static std::mutex mu;
     static std::map<uint64_t, std::vector<int>> done;  // at most the smooth lengths up to 2^15
@@ -185,7 +193,8 @@ std::vector<int> mix_schedule(uint64_t n) {
         std::sort(r.begin(), r.end());
         do {
             double score = r.size() < 2 ? 1.0
-                                        : best_shape(P_F32, n, r, 1u << 30, false, false, kLdsBudget, 0, 0, false, nullptr);
+                                        : best_shape(P_F32, n, r, 1u << 30, false, false, kLdsBudget, 0, 0, false,
+                                                     false, nullptr);
             if (score <= 0) score = 1e-3;
             const double v = s.first / score * (r.front() < r.back() ? 1.02 : 1.0) * (r.front() < r[r.size() > 1] ? 1.01 : 1.0);
             if (v < value) {
@@ -199,7 +208,7 @@ std::vector<int> mix_schedule(uint64_t n) {
 }
 
 bool mix_plan(int arith, uint64_t n, uint64_t lines, bool ld_lf, bool st_lf, size_t budget, uint32_t fixed_nt,
-              uint32_t forced_lpw, Mix* out) {
+              uint32_t forced_lpw, bool real, Mix* out) {
     const std::vector<int> rad = mix_schedule(n);
     if (rad.size() < 2 || !lines) return false;
     // batched tiles: the launch's LDS is its largest tile's, so half the
@@ -207,7 +216,7 @@ bool mix_plan(int arith, uint64_t n, uint64_t lines, bool ld_lf, bool st_lf, siz
     // (several rounds per middle stage) only where nothing else does
     for (int pp = 0; pp < 2; pp++)
         for (size_t b : {fixed_nt ? budget / 2 : budget, budget})
-            if (best_shape(arith, n, rad, lines, ld_lf, st_lf, b, fixed_nt, forced_lpw, pp, out) > 0) return true;
+            if (best_shape(arith, n, rad, lines, ld_lf, st_lf, b, fixed_nt, forced_lpw, pp, real, out) > 0) return true;
     return false;
 }
 

@@ -576,6 +576,18 @@ struct Builder {
         return t;
     }
 
+    // W_n^k for k <= n / 4 (the bin pairs of half-length real lines), f32.
+    const void* half_twiddles(uint64_t n) {
+        const std::string key = "h" + std::to_string(n);
+        auto it = tw_cache.find(key);
+        if (it != tw_cache.end()) return it->second;
+        const uint64_t cnt = n / 4 + 1;
+        void* t = alloc(cnt * sizeof(cpx<float>), "roots prec=f32 n=" + std::to_string(n) + " count=" + std::to_string(cnt));
+        hip_check(gen_twiddles(P_F32, t, n, cnt, s), "half-length twiddles");
+        tw_cache[key] = t;
+        return t;
+    }
+
     static std::vector<int> parse_radices(const char* s) {
         std::vector<int> r;
         int v = 0;
@@ -635,9 +647,17 @@ struct Builder {
         return best;
     }
 
+    // Line stride of the real side of a contiguous real line op: n real
+    // elements, or n / 2 complex ones at half length.
+    static void set_real_side(Op& op, uint64_t stride) {
+        if (op.ldm == LD_REAL) op.a.in_so = (int64_t)stride;
+        else if (op.ldm == LD_HERMITIAN) op.a.out_so = (int64_t)stride;
+    }
+
     // Makes `op` (lines, lane layout and modes set) a runtime-schedule line
     // op: the register form (mix_kernels.hpp) for complex lines of at least two
-    // stages, else the LDS-to-LDS one.  The radix schedule depends on the
+    // stages and even real lines of twice that, else (short or odd real
+    // lines) the LDS-to-LDS one.  The radix schedule depends on the
     // length alone, so a line's result does not depend on its neighbours or on
     // the tile.
     void runtime_schedule(Op& op, bool batched, uint32_t forced_lpw) {
@@ -647,14 +667,23 @@ struct Builder {
         const uint64_t n = op.n;
         const size_t es = elem_bytes(P.arith);
         const uint32_t fit = (uint32_t)(P.lds_budget / (2 * lds_line_stride((uint32_t)n) * es));
-        if (op.ldm == LD_COMPLEX && op.stm == ST_COMPLEX) {
+        set_real_side(op, n);
+        // even real lines run at half length
+        const bool real = op.ldm == LD_REAL || op.ldm == LD_HERMITIAN;
+        const uint64_t m = real ? n / 2 : n;
+        if (!real || (n % 2 == 0 && op.a.S1 == 1 && op.a.S2 == 1 && P.prec == P_F32)) {
             bool ok = false;
             for (uint32_t lpw = forced_lpw; !ok; lpw--) {
-                ok = mix_plan(P.arith, n, op.a.lines, op.ld_lf, op.st_lf, P.lds_budget, batched ? 256 : 0, lpw, &op.mix);
+                ok = mix_plan(P.arith, m, op.a.lines, op.ld_lf, op.st_lf, P.lds_budget, batched ? 256 : 0, lpw, real,
+                              &op.mix);
                 if (lpw <= 1) break;
             }
             if (ok) {
-                op.a.tw = stage_twiddles(P.arith, mix_schedule(n));
+                op.a.tw = stage_twiddles(P.arith, mix_schedule(m));
+                if (real) {
+                    set_real_side(op, m);
+                    op.a.half_tw = half_twiddles(n);
+                }
                 return;
             }
             op.mix = Mix{};
@@ -761,9 +790,9 @@ struct Builder {
             if (rv->persist) d << " pipe" << rv->persist;
         } else {
             runtime_schedule(op, P.batch_mode, forced_lpw);
-            d << "lds N=" << n << " " << (op.mix.ns ? radices_str(mix_schedule(n)) : sched_str(op.sc))
+            d << "lds N=" << n << " " << (op.mix.ns ? radices_str(mix_schedule(op.mix.n)) : sched_str(op.sc))
               << " lines=" << ls.lines << " lpw=" << (op.mix.ns ? op.mix.lpw : op.sc.lpw);
-            if (op.mix.ns) d << " nt=" << op.mix.nt << (op.mix.pp ? " pp" : "");
+            if (op.mix.ns) d << " nt=" << op.mix.nt << (op.mix.pp ? " pp" : "") << (op.mix.pairs ? " half" : "");
         }
         if (ld_lf || st_lf) d << (ld_lf ? " ldLF" : "") << (st_lf ? " stLF" : "");
         if (post) d << " post";
@@ -2260,6 +2289,8 @@ int autotune_sequence(const mifft_config* cfgs, const mifft_kind* kinds, int cou
                 Op c = *ref;
                 c.kind = OP_REG;
                 c.rv = v;
+                c.mix = Mix{};
+                if (!c.fold) Builder::set_real_side(c, c.n);
                 c.a.tw = TB.stage_twiddles(T.arith, Builder::parse_radices(v->radices));
                 cands.emplace_back(reg_variant_name(v), c);
             }
@@ -2282,6 +2313,8 @@ int autotune_sequence(const mifft_config* cfgs, const mifft_kind* kinds, int cou
                             o.sc = c.sc;
                             o.mix = c.mix;
                             o.a.tw = c.a.tw;
+                            o.a.half_tw = c.a.half_tw;
+                            if (!o.fold) Builder::set_real_side(o, c.mix.pairs ? c.mix.n : o.n);
                         }
             };
             hip_check(hipStreamSynchronize(s), "autotune tables");
