@@ -77,7 +77,7 @@ __device__ __forceinline__ LineBase line_base(const LineArgs& a, uint32_t g) {
 __device__ __forceinline__ double2 post_f64(const LineArgs& a, uint64_t t) {
     const vd2_t h = gptr<vd2_t>(a.post_hi)[t >> a.post_shift];
     const vd2_t l = gptr<vd2_t>(a.post_lo)[t & a.post_mask];
-    return make_double2(h.x * l.x - h.y * l.y, h.x * l.y + h.y * l.x);
+    return make_double2(fma(h.x, l.x, -(h.y * l.y)), fma(h.x, l.y, h.y * l.x));
 }
 
 // W_P^t rounded once from that product.
@@ -100,7 +100,7 @@ struct PostSeq {
     template <class T>
     __device__ __forceinline__ cpx<T> next() {
         const cpx<T> r = mk<T>((T)w.x, (T)w.y);
-        w = make_double2(w.x * step.x - w.y * step.y, w.x * step.y + w.y * step.x);
+        w = make_double2(fma(w.x, step.x, -(w.y * step.y)), fma(w.x, step.y, w.y * step.x));
         return r;
     }
 };
@@ -792,10 +792,10 @@ __device__ __forceinline__ void prime_acc(cpx<T>& A, cpx<T>& B, const cpx<T>* ap
         constexpr int e = (m * q) % R;
         constexpr T c = (T)root_cos<R>(e);
         constexpr T sn = (T)root_sin<R>(e);
-        A.x += c * ap[m - 1].x;
-        A.y += c * ap[m - 1].y;
-        B.x += sn * am[m - 1].x;
-        B.y += sn * am[m - 1].y;
+        A.x = fma(c, ap[m - 1].x, A.x);
+        A.y = fma(c, ap[m - 1].y, A.y);
+        B.x = m == 1 ? sn * am[0].x : fma(sn, am[m - 1].x, B.x);
+        B.y = m == 1 ? sn * am[0].y : fma(sn, am[m - 1].y, B.y);
         prime_acc<R, q, m + 1, T>(A, B, ap, am);
     }
 }

@@ -11,6 +11,11 @@
 
 #include "roots.hpp"
 
+// Fused multiply-adds are written out (fma) and never formed by the compiler:
+// which of two products it would fuse depends on the code around them, and a
+// line's result must not depend on the tile shape, unroll or kernel that runs it.
+#pragma clang fp contract(off)
+
 namespace mifft {
 
 template <class T>
@@ -36,12 +41,12 @@ __device__ __forceinline__ cpx<T> operator-(cpx<T> a, cpx<T> b) {
 // a * b
 template <class T>
 __device__ __forceinline__ cpx<T> cmul(cpx<T> a, cpx<T> b) {
-    return mk<T>(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
+    return mk<T>(fma(a.x, b.x, -(a.y * b.y)), fma(a.x, b.y, a.y * b.x));
 }
 // a * conj(b)
 template <class T>
 __device__ __forceinline__ cpx<T> cmulc(cpx<T> a, cpx<T> b) {
-    return mk<T>(a.x * b.x + a.y * b.y, a.y * b.x - a.x * b.y);
+    return mk<T>(fma(a.x, b.x, a.y * b.y), fma(a.y, b.x, -(a.x * b.y)));
 }
 // -i * a
 template <class T>
@@ -228,7 +233,7 @@ __device__ __forceinline__ cpx<T> twc(cpx<T> v) {
         constexpr T c = (T)root_cos<R>(tt);
         constexpr T s = (T)root_sin<R>(tt);
         // (x + iy)(c - is)
-        return mk<T>(v.x * c + v.y * s, v.y * c - v.x * s);
+        return mk<T>(fma(v.x, c, v.y * s), fma(v.y, c, -(v.x * s)));
     }
 }
 
@@ -275,10 +280,10 @@ struct DftOdd {
             constexpr int m = (j * k) % R;
             constexpr T c = (T)root_cos<R>(m);
             constexpr T s = (T)root_sin<R>(m);
-            A.x += c * a[j - 1].x;
-            A.y += c * a[j - 1].y;
-            B.x += s * b[j - 1].x;
-            B.y += s * b[j - 1].y;
+            A.x = fma(c, a[j - 1].x, A.x);
+            A.y = fma(c, a[j - 1].y, A.y);
+            B.x = j == 1 ? s * b[0].x : fma(s, b[j - 1].x, B.x);
+            B.y = j == 1 ? s * b[0].y : fma(s, b[j - 1].y, B.y);
             acc<k, j + 1>(A, B, a, b);
         }
     }
@@ -308,8 +313,18 @@ struct DftOdd {
     }
 };
 
+// X_1, X_2 = (v_0 - a / 2) -+ i sin(pi/3) b: 12 instructions.
 template <class T>
-struct Dft<3, T> : DftOdd<3, T> {};
+struct Dft<3, T> {
+    static __device__ __forceinline__ void run(cpx<T>* v) {
+        constexpr T c = (T)root_cos<3>(1), s = (T)root_sin<3>(1);
+        const cpx<T> a = v[1] + v[2], b = v[1] - v[2];
+        const cpx<T> m = mk<T>(fma(c, a.x, v[0].x), fma(c, a.y, v[0].y));
+        v[0] = v[0] + a;
+        v[1] = mk<T>(fma(s, b.y, m.x), fma(-s, b.x, m.y));
+        v[2] = mk<T>(fma(-s, b.y, m.x), fma(s, b.x, m.y));
+    }
+};
 template <class T>
 struct Dft<5, T> : DftOdd<5, T> {};
 template <class T>
@@ -389,14 +404,83 @@ struct DftCoprime {
     }
 };
 
+// Radix-4 butterfly of z0, W_8 z1, W_8^2 z2, W_8^3 z3: the multiples of
+// sqrt(1/2) fold into the last additions (20 instructions, where the
+// twiddles and a plain radix-4 butterfly take 24).
 template <class T>
-struct Dft<8, T> : DftComp<2, 4, T> {};
+__device__ __forceinline__ void dft4_w8(cpx<T>& z0, cpx<T>& z1, cpx<T>& z2, cpx<T>& z3) {
+    constexpr T h = (T)0.707106781186547524400844362104849039;
+    const cpx<T> a0 = mk<T>(z0.x + z2.y, z0.y - z2.x), a1 = mk<T>(z0.x - z2.y, z0.y + z2.x);
+    const cpx<T> p = z1 - z3, q = z1 + z3;
+    const cpx<T> u = mk<T>(p.x + q.y, p.y - q.x), w = mk<T>(p.x - q.y, p.y + q.x);
+    z0 = mk<T>(fma(h, u.x, a0.x), fma(h, u.y, a0.y));
+    z2 = mk<T>(fma(-h, u.x, a0.x), fma(-h, u.y, a0.y));
+    z1 = mk<T>(fma(-h, w.x, a1.x), fma(-h, w.y, a1.y));
+    z3 = mk<T>(fma(h, w.x, a1.x), fma(h, w.y, a1.y));
+}
+
+// Radix 8: two radix-4 butterflies over the sums and differences v_n +- v_{n+4}.
 template <class T>
-struct Dft<16, T> : DftComp<4, 4, T> {};
+struct Dft<8, T> {
+    static __device__ __forceinline__ void run(cpx<T>* v) {
+        cpx<T> e[4], o[4];
+#pragma unroll
+        for (int n = 0; n < 4; n++) {
+            e[n] = v[n] + v[n + 4];
+            o[n] = v[n] - v[n + 4];
+        }
+        Dft<4, T>::run(e);
+        dft4_w8(o[0], o[1], o[2], o[3]);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            v[2 * k] = e[k];
+            v[2 * k + 1] = o[k];
+        }
+    }
+};
+
+// Radix 16 as 4 x 4: column k1 holds z_n2 = W_16^(n2 k1) y_n2[k1].  For k1 = 1
+// and 3 the middle twiddle is an odd multiple of pi/4 and folds into the
+// additions that follow it; k1 = 2 is dft4_w8.
 template <class T>
-struct Dft<32, T> : DftComp<4, 8, T> {};
-template <class T>
-struct Dft<64, T> : DftComp<8, 8, T> {};
+struct Dft<16, T> {
+    template <int k1>
+    static __device__ __forceinline__ void odd(cpx<T>* z) {
+        constexpr T h = (T)0.707106781186547524400844362104849039;
+        z[1] = twc<16, k1>(z[1]);
+        z[3] = twc<16, 3 * k1>(z[3]);
+        // z2 W_16^(2 k1) = h u
+        const cpx<T> u = k1 == 1 ? mk<T>(z[2].x + z[2].y, z[2].y - z[2].x) : mk<T>(z[2].y - z[2].x, -z[2].x - z[2].y);
+        const cpx<T> a0 = mk<T>(fma(h, u.x, z[0].x), fma(h, u.y, z[0].y));
+        const cpx<T> a1 = mk<T>(fma(-h, u.x, z[0].x), fma(-h, u.y, z[0].y));
+        const cpx<T> a2 = z[1] + z[3], a3 = mul_mi(z[1] - z[3]);
+        z[0] = a0 + a2;
+        z[2] = a0 - a2;
+        z[1] = a1 + a3;
+        z[3] = a1 - a3;
+    }
+    static __device__ __forceinline__ void run(cpx<T>* v) {
+        cpx<T> y[4][4], z[4][4];
+#pragma unroll
+        for (int n2 = 0; n2 < 4; n2++) {
+#pragma unroll
+            for (int n1 = 0; n1 < 4; n1++) y[n2][n1] = v[4 * n1 + n2];
+            Dft<4, T>::run(y[n2]);
+        }
+#pragma unroll
+        for (int k1 = 0; k1 < 4; k1++)
+#pragma unroll
+            for (int n2 = 0; n2 < 4; n2++) z[k1][n2] = y[n2][k1];
+        Dft<4, T>::run(z[0]);
+        odd<1>(z[1]);
+        dft4_w8(z[2][0], z[2][1], z[2][2], z[2][3]);
+        odd<3>(z[3]);
+#pragma unroll
+        for (int k1 = 0; k1 < 4; k1++)
+#pragma unroll
+            for (int k2 = 0; k2 < 4; k2++) v[k1 + 4 * k2] = z[k1][k2];
+    }
+};
 template <class T>
 struct Dft<6, T> : DftCoprime<2, 3, T> {};
 template <class T>

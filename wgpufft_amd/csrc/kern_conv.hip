@@ -123,10 +123,10 @@ __global__ void __launch_bounds__(256) k_direct_prime(LineArgs a, uint32_t p, ui
             if (t >= p) t -= p;
             const cpx<float> u = x[n], v = x[p - n];
             const float c = w[t].x, sn = -w[t].y;  // W_p^t = cos - i sin
-            ar += (u.x + v.x) * c;
-            ai += (u.y + v.y) * c;
-            br += (u.x - v.x) * sn;
-            bi += (u.y - v.y) * sn;
+            ar = fma(u.x + v.x, c, ar);
+            ai = fma(u.y + v.y, c, ai);
+            br = fma(u.x - v.x, sn, br);
+            bi = fma(u.y - v.y, sn, bi);
         }
         // -i B = (B.y, -B.x)
         store_point<FmtF32, ST_COMPLEX, false>(a, b.out, b.j, k, p, mk<float>(x0.x + ar + bi, x0.y + ai - br));

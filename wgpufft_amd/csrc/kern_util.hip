@@ -226,7 +226,7 @@ __global__ void k_real_part(const float2* __restrict__ full, float* __restrict__
 __device__ __forceinline__ float2 half_twiddle(const double2* hi, const double2* lo, uint32_t sh, uint32_t mask,
                                                uint32_t k) {
     const double2 a = hi[k >> sh], b = lo[k & mask];
-    return make_float2((float)(a.x * b.x - a.y * b.y), (float)(a.x * b.y + a.y * b.x));
+    return make_float2((float)fma(a.x, b.x, -(a.y * b.y)), (float)fma(a.x, b.y, a.y * b.x));
 }
 
 __global__ void k_r2c_post(const float2* __restrict__ z, float2* __restrict__ x, uint32_t h, uint64_t lines, float sc,
@@ -242,7 +242,7 @@ __global__ void k_r2c_post(const float2* __restrict__ z, float2* __restrict__ x,
         const float2 d = make_float2(a.x - b.x, a.y + b.y);  // Z[k] - conj Z[h-k]
         const float2 B = make_float2(0.5f * d.y, -0.5f * d.x);  // d / (2i)
         const float2 w = half_twiddle(hi, lo, sh, mask, k);
-        const float2 r = make_float2(A.x + w.x * B.x - w.y * B.y, A.y + w.x * B.y + w.y * B.x);
+        const float2 r = make_float2(fma(-w.y, B.y, fma(w.x, B.x, A.x)), fma(w.y, B.x, fma(w.x, B.y, A.y)));
         x[e] = make_float2(r.x * sc, r.y * sc);
     }
 }
@@ -263,7 +263,7 @@ __global__ void k_c2r_pre(const float2* __restrict__ x, float2* __restrict__ z, 
         const float2 E = make_float2(a.x + b.x, a.y - b.y);   // X[k] + conj X[h-k]
         const float2 d = make_float2(a.x - b.x, a.y + b.y);   // X[k] - conj X[h-k]
         const float2 w = half_twiddle(hi, lo, sh, mask, k);  // W^k; O = d conj(W^k)
-        const float2 O = make_float2(d.x * w.x + d.y * w.y, d.y * w.x - d.x * w.y);
+        const float2 O = make_float2(fma(d.x, w.x, d.y * w.y), fma(d.y, w.x, -(d.x * w.y)));
         z[e] = make_float2(E.x - O.y, E.y + O.x);
     }
 }

@@ -14,7 +14,7 @@ namespace mifft {
 // pairs for odd primes, two factors for composites, without a twiddle between
 // coprime ones).
 static double butterfly_ops(int r) {
-    static const double ops[17] = {0, 0, 4, 14, 16, 36, 40, 66, 56, 100, 92, 150, 104, 204, 160, 178, 160};
+    static const double ops[17] = {0, 0, 4, 12, 16, 36, 36, 66, 52, 88, 92, 150, 96, 204, 160, 168, 152};
     return ops[r];
 }
 // Work of one stage per point: the butterfly, and in the same unit the
