@@ -122,3 +122,54 @@ def test_half_length_real_volume(torch_cuda):
     assert oracle.rel_l2(y, np.fft.rfftn(x.astype(np.float64), axes=(1, 2, 3)).reshape(-1)) <= 1e-6
     z = run(c2r, y, x.nbytes).view(np.float32)
     assert oracle.rel_l2(z, x.astype(np.float64).reshape(-1)) <= 1e-6
+
+
+@pytest.mark.parametrize("p,batch", [(29, 1), (29, 300), (61, 77), (73, 5), (127, 64), (257, 9), (1009, 7), (2003, 2),
+                                     (4051, 1), (7561, 3)])
+def test_rader_register_convolution(torch_cuda, p, batch):
+    """Cyclic Rader lines on the register stages, contiguous and strided."""
+    for inverse in (False, True):
+        x = seeded_complex(p + batch, p * batch)
+        plan = FftPlan.c2c((FftConfig.inverse(p) if inverse else FftConfig.new(p)).with_batch(batch))
+        assert plan.describe().startswith("rader") and " nt=" in plan.describe(), plan.describe()
+        e = oracle.rel_l2(run(plan, x, x.nbytes), c2c_expected(x, [p], batch=batch, inverse=inverse))
+        assert e <= 1e-6, (p, batch, inverse, e)
+    width = 3 if p > 2000 else 19
+    x = seeded_complex(p, p * width)
+    plan = FftPlan.c2c(FftConfig.new_nd([width, p]).with_axes([1]))
+    want = np.fft.fft(x.astype(np.complex128).reshape(p, width), axis=0).reshape(-1)
+    assert oracle.rel_l2(run(plan, x, x.nbytes), want) <= 1e-6, (p, plan.describe())
+
+
+@pytest.mark.parametrize("n,kind", [(127, "rader"), (1019, "rader"), (3001, "rader"), (34, "bluestein"),
+                                    (611, "bluestein"), (1622, "bluestein")])
+def test_double_precision_convolutions(torch_cuda, n, kind):
+    for prec, bound in ((FftPrecision.F64, 1e-13), (FftPrecision.Df64, 1e-11)):
+        batch = 6
+        v = np.random.default_rng(n).uniform(-1, 1, (n * batch, 2)).astype(np.float32).astype(np.float64)
+        plan = FftPlan.c2c(FftConfig.new(n).with_batch(batch).with_precision(prec))
+        assert plan.describe().startswith(kind) and " nt=" in plan.describe(), plan.describe()
+        if prec == FftPrecision.F64:
+            got = run(plan, v.reshape(-1), v.nbytes).reshape(-1, 2)
+        else:
+            w = np.stack([v, np.zeros_like(v)], -1).astype(np.float32)
+            w = run(plan, w.reshape(-1), v.nbytes).reshape(-1, 2, 2).astype(np.float64)
+            got = w[..., 0] + w[..., 1]
+        want = np.fft.fft((v[:, 0] + 1j * v[:, 1]).reshape(batch, n)).reshape(-1)
+        e = oracle.rel_l2(got[:, 0] + 1j * got[:, 1], want)
+        assert e <= bound, (n, prec, e)
+
+
+def test_batched_convolutions_equal_standalone(torch_cuda):
+    import torch
+    items, want = [], []
+    for k, (n, b) in enumerate([(29, 40), (127, 9), (257, 3), (1009, 5), (2003, 2)]):
+        x = seeded_complex(200 + k, n * b)
+        cfg = FftConfig.new(n).with_batch(b)
+        want.append(run(FftPlan.c2c(cfg), x, x.nbytes))
+        items.append(dict(n=n, batch=b, input=to_dev(x), output=empty_dev(x.nbytes)))
+    FftBatch(items).execute()
+    torch.cuda.synchronize()
+    for it, w in zip(items, want):
+        got = from_dev(it["output"], np.complex64)
+        assert np.array_equal(got.view(np.uint32), w.view(np.uint32)), it["n"]

@@ -17,7 +17,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libmifft.so")
-SOURCES = ["kern_line.hip", "kern_mix_f32.hip", "kern_mix_f64.hip", "kern_mix_df64.hip", "kern_mix_real.hip", "kern_conv.hip", "kern_regconv.hip", "kern_util.hip", "kern_batch.hip", "kern_small.hip", "scratch.hip", "plan.cpp", "mix_plan.cpp",
+SOURCES = ["kern_line.hip", "kern_mix_f32.hip", "kern_mix_f64.hip", "kern_mix_df64.hip", "kern_mix_real.hip",
+           "kern_mix_conv_f32.hip", "kern_mix_conv_f64.hip", "kern_mix_conv_df64.hip", "kern_conv.hip", "kern_regconv.hip", "kern_util.hip", "kern_batch.hip", "kern_small.hip", "scratch.hip", "plan.cpp", "mix_plan.cpp",
            "api.cpp", "diagnostics.cpp", "batch.cpp", "serve.cpp", "cpu_plan.cpp", "cpu_fft_avx2.cpp", "cpu_fft_base.cpp"]
 # Host-only translation units of the CPU FFT engine: plain C++ (no device
 # code), one built for AVX2 + FMA and one for the x86-64 baseline; the library
@@ -27,9 +28,13 @@ ARCH = os.environ.get("MIFFT_ARCH", "gfx950")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 CXX = os.environ.get("CXX", "g++")
-# Packed-FP32 instructions are disabled for every HIP translation unit.
+# Packed-FP32 instructions are disabled for every HIP translation unit.  The
+# user limit lets large kernels read their by-value arguments from the kernel
+# argument segment: above its default of 300 uses the compiler copies the whole
+# struct to scratch first.
 COMMON = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-Wall",
           "-Wno-unused-result", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+          "-mllvm", "-instcombine-max-copied-from-constant-users=20000",
           "-I", os.path.join(HERE, "..", "include")]
 
 

@@ -229,12 +229,27 @@ void batch_build(const BatchEntry* entries, int32_t count, char* ws_base, BatchB
                     break;
                 case OP_RADER:
                 case OP_BLUESTEIN:
-                    if (f64) cls = op.kind == OP_RADER ? BC_RADER_F64 : BC_BLUESTEIN_F64;
+                    if (op.conv.mix)
+                        cls = op.kind == OP_RADER ? (f64 ? BC_MIX_RADER_F64 : BC_MIX_RADER)
+                                                  : (f64 ? BC_MIX_BLUESTEIN_F64 : BC_MIX_BLUESTEIN);
+                    else if (f64) cls = op.kind == OP_RADER ? BC_RADER_F64 : BC_BLUESTEIN_F64;
                     else if (op.kind == OP_RADER) cls = sched_has_medium_prime(op.conv.sc) ? BC_RADER_MED : BC_RADER;
                     else cls = BC_BLUESTEIN;
                     d.conv = op.conv;
-                    lpw = op.conv.sc.lpw;
-                    op_lds = conv_kernel_bytes(op.prec, op.conv.m, op.conv.sc.lpw);
+                    if (op.conv.mix) {
+                        // a plan made for one line: the tile for all lines that run it
+                        MixConv m;
+                        if (e.mult > 1 && mix_conv_plan(P.arith, op.conv.m, (uint64_t)op.conv.io.lines * e.mult,
+                                                        op.conv.mx.f.ld_lf, op.conv.mx.f.st_lf, P.lds_budget, 256, &m)) {
+                            m.rtw = op.conv.mx.rtw;
+                            d.conv.mx = m;
+                        }
+                        lpw = d.conv.mx.f.lpw;
+                        op_lds = mix_conv_lds_bytes(P.arith, d.conv.mx);
+                    } else {
+                        lpw = op.conv.sc.lpw;
+                        op_lds = conv_kernel_bytes(op.prec, op.conv.m, op.conv.sc.lpw);
+                    }
                     if (op.rcv) {
                         // the register Bluestein kernel's own class (same tile body)
                         cls = regb_batch_class(op.rcv->m);

@@ -67,6 +67,10 @@ enum BatchClass : uint32_t {
     BC_MIX_POST_F64,
     BC_MIX_R2C,  // even real lines at half length
     BC_MIX_C2R,
+    BC_MIX_RADER,  // convolutions of a runtime schedule (mix_conv.hpp)
+    BC_MIX_RADER_F64,
+    BC_MIX_BLUESTEIN,
+    BC_MIX_BLUESTEIN_F64,
     BC_COUNT
 };
 

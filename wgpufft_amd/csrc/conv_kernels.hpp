@@ -24,11 +24,6 @@
 
 namespace mifft {
 
-// Primes above this stage their lines through LDS in natural order (for
-// N = 1009 over 1 GiB 21 % faster; for N = 17, whose line spans three cache
-// lines, 18 % slower than gathering straight from memory).
-constexpr uint32_t kRaderStagedMin = 64;
-
 // Rader's filter step on the forward spectra in LDS: keeps bin 0 (the sum
 // of the permuted inputs) in s0 and leaves swap(A[k] F[k]) for the inverse.
 template <class T>
@@ -44,7 +39,9 @@ __device__ __forceinline__ void rader_filter(const ConvArgs& c, cpx<T>* r, cpx<T
     }
 }
 
-// MED: the schedule holds medium prime radices (17..61), f32 only.
+// The LDS-to-LDS form: convolutions of at most 16 points (one stage), and with
+// MED the schedules that hold medium prime radices (17..61, f32 only); the
+// others run on the register stages (mix_conv.hpp).
 template <class Fmt, bool MED = false>
 __device__ __forceinline__ void rader_tile(const ConvArgs& c, unsigned char* smem_raw, uint32_t g0) {
     using T = typename Fmt::T;
@@ -56,15 +53,14 @@ __device__ __forceinline__ void rader_tile(const ConvArgs& c, unsigned char* sme
     cpx<T>* bufB = bufA + lpw * lstr;
     cpx<T>* x0 = bufB + lpw * lstr;  // lpw entries
     cpx<T>* s0 = x0 + lpw;           // lpw entries
-    // Long lines: the line in natural order into bufB (coalesced loads),
+    // Long lines (MED): the line in natural order into bufB (coalesced loads),
     // then the gather a[q] = x[g^q] (zero-padded to M) and x0 = x[0] from
     // LDS, so that no global load waits on the permutation table's.  Short
     // lines (a few cache lines each) gather straight from memory.  Lines
     // past the end read the last line and are never stored.
     const uint32_t total = lpw * M;
     const uint32_t tpl = slot_tpl(lpw), slots = tpl * lpw;
-    const bool staged = p > kRaderStagedMin;
-    if (staged) {
+    if constexpr (MED) {
         for (uint32_t s = threadIdx.x; s < slots; s += blockDim.x) {
             const LineSlot m = line_slot(s, lpw, tpl, sc.ld_lf);
             const uint32_t g = g0 + m.l;
@@ -144,7 +140,7 @@ __device__ __forceinline__ void rader_tile(const ConvArgs& c, unsigned char* sme
     // X[g^-u] = x0 + c[u], X[0] = x0 + sum a.  Long lines: permuted in LDS
     // (into the buffer the second transform did not end in), then stored in
     // natural order (coalesced); short lines: scattered straight to memory.
-    if (staged) {
+    if constexpr (MED) {
         cpx<T>* y = (r2 == bufA) ? bufB : bufA;
         for (uint32_t e = threadIdx.x; e < lpw * p; e += blockDim.x) {
             const uint32_t l = fdiv(e, c.dn);

@@ -15,7 +15,7 @@
 // This is the gfx950 counterpart of recording many plans into one shared
 // compute pass with FftRecorder (src/plan.rs:38-95, src/runtime/recorder.rs).
 #include "batch_kernels.hpp"
-#include "mix_kernels.hpp"
+#include "mix_conv.hpp"
 #include "reg_conv.hpp"
 
 namespace mifft {
@@ -91,6 +91,11 @@ __device__ __noinline__ uint32_t mix_tiles(MIFFT_TILE_ARGS) {
         mix_tile<Fmt, LD_COMPLEX, ST_COMPLEX, POST>(d.a, d.mix, smem, g0);
     });
 }
+template <class Fmt, bool RADER>
+__device__ __noinline__ uint32_t mix_conv_tiles(MIFFT_TILE_ARGS) {
+    return tile_run(tiles, ntiles, counter, ops, t,
+                    [&](const OpDesc& d, uint32_t g0) { mix_conv_tile<Fmt, RADER>(d.conv, smem, g0); });
+}
 template <bool C2R>
 __device__ __noinline__ uint32_t mix_real_tiles(MIFFT_TILE_ARGS) {
     return tile_run(tiles, ntiles, counter, ops, t,
@@ -158,6 +163,10 @@ __global__ void __launch_bounds__(256, 4) k_batch(const BatchTile* __restrict__ 
             case BC_MIX_POST_F64: t = mix_tiles<FmtF64, true>(MIFFT_TILE_PASS); break;
             case BC_MIX_R2C: t = mix_real_tiles<false>(MIFFT_TILE_PASS); break;
             case BC_MIX_C2R: t = mix_real_tiles<true>(MIFFT_TILE_PASS); break;
+            case BC_MIX_RADER: t = mix_conv_tiles<FmtF32, true>(MIFFT_TILE_PASS); break;
+            case BC_MIX_RADER_F64: t = mix_conv_tiles<FmtF64, true>(MIFFT_TILE_PASS); break;
+            case BC_MIX_BLUESTEIN: t = mix_conv_tiles<FmtF32, false>(MIFFT_TILE_PASS); break;
+            case BC_MIX_BLUESTEIN_F64: t = mix_conv_tiles<FmtF64, false>(MIFFT_TILE_PASS); break;
             case BC_RADER: t = rader_tiles<FmtF32>(MIFFT_TILE_PASS); break;
             case BC_BLUESTEIN: t = bluestein_tiles<FmtF32>(MIFFT_TILE_PASS); break;
             case BC_RADER_F64: t = rader_tiles<FmtF64>(MIFFT_TILE_PASS); break;

@@ -1,0 +1,9 @@
+#include "mix_conv.hpp"
+
+namespace mifft {
+
+hipError_t launch_mix_conv_f32(bool rader, const ConvArgs& c, hipStream_t s) {
+    return launch_mix_conv_fmt<FmtF32>(rader, c, s);
+}
+
+}  // namespace mifft

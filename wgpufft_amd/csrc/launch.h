@@ -68,7 +68,7 @@ constexpr size_t kLdsBudget = 160 * 1024;
 // Runtime-schedule register line kernels (mix_kernels.hpp, kern_mix.hip): the
 // schedule and tile shape of one length (mix_plan.cpp).  Counts are in
 // elements; the d* fields are mix_div multipliers.
-constexpr int kMixStages = 8;
+constexpr int kMixStages = 6;  // enough for every length up to 2^15
 struct MixStage {
     uint32_t code;      // radix + 32 * unroll
     uint32_t nr, nrp;   // butterflies per line and their LDS pitch (odd)
@@ -107,20 +107,44 @@ inline hipError_t launch_mix(int prec, int ldm, int stm, int post, const LineArg
                            : launch_mix_df64(ldm, stm, post, a, mx, s);
 }
 
+// The two transforms of a fused convolution: the second one's schedule is the
+// first one's reversed, with the same lines, threads and LDS pitch.
+struct MixConv {
+    Mix f, r;
+    const void* rtw;  // stage twiddles of the reversed schedule
+};
+bool mix_conv_plan(int arith, uint64_t m, uint64_t lines, bool ld_lf, bool st_lf, size_t budget, uint32_t fixed_nt,
+                   MixConv* out);
+size_t mix_conv_lds_bytes(int arith, const MixConv& x);
+
 // Fused Rader / Bluestein convolution kernels (one line per workgroup pass).
 struct ConvArgs {
     LineArgs io;              // the prime / Bluestein line layout (n points)
-    Sched sc;                 // schedule of the convolution length M
+    // schedule of the convolution length M: sc, or mx for the register form
+    union {
+        Sched sc{};
+        MixConv mx;
+    };
     const void* filt;         // FFT_M of the filter, scaled by 1/M (arith type)
     const void* chirp;        // Bluestein chirp c[n] (arith type), or nullptr
     const uint32_t* perm_in;  // Rader gather g^q mod p, q < p-1
     const uint32_t* perm_out; // Rader scatter g^-u mod p, u < p-1
     uint32_t n;               // transform length
     uint32_t m;               // convolution length
+    uint32_t mix;             // 1: the register form
     DivMagic dn;              // divide by n (Rader)
 };
 hipError_t launch_rader(int prec, const ConvArgs& c, hipStream_t s);
 hipError_t launch_bluestein(int prec, const ConvArgs& c, hipStream_t s);
+// The register forms (mix_conv.hpp, kern_mix_conv_*.hip).
+hipError_t launch_mix_conv_f32(bool rader, const ConvArgs& c, hipStream_t s);
+hipError_t launch_mix_conv_f64(bool rader, const ConvArgs& c, hipStream_t s);
+hipError_t launch_mix_conv_df64(bool rader, const ConvArgs& c, hipStream_t s);
+inline hipError_t launch_mix_conv(int prec, bool rader, const ConvArgs& c, hipStream_t s) {
+    return prec == P_F32   ? launch_mix_conv_f32(rader, c, s)
+           : prec == P_F64 ? launch_mix_conv_f64(rader, c, s)
+                           : launch_mix_conv_df64(rader, c, s);
+}
 // Register-resident f32 Bluestein kernels (reg_conv.hpp, kern_regconv.hip),
 // one per power-of-two convolution length M: `lines` lines of `tpl` threads
 // per workgroup, radix schedule `radices` (stage twiddles in that format).

@@ -220,4 +220,30 @@ bool mix_plan(int arith, uint64_t n, uint64_t lines, bool ld_lf, bool st_lf, siz
     return false;
 }
 
+size_t mix_conv_lds_bytes(int arith, const MixConv& x) {
+    // two more elements per line: Rader's x[0] and its sum of inputs
+    return mix_lds_bytes(arith, x.f) + 2 * (size_t)x.f.lpw * (arith == P_F32 ? 8 : 16);
+}
+
+bool mix_conv_plan(int arith, uint64_t m, uint64_t lines, bool ld_lf, bool st_lf, size_t budget, uint32_t fixed_nt,
+                   MixConv* out) {
+    const std::vector<int> rad = mix_schedule(m);
+    if (rad.size() < 2 || !lines) return false;
+    const std::vector<int> rev(rad.rbegin(), rad.rend());
+    for (int pp = 0; pp < 2; pp++)
+        for (size_t b : {fixed_nt ? budget / 2 : budget, budget}) {
+            Mix f;
+            // (the two extra elements per line fit what a pitch above m leaves)
+            if (best_shape(arith, m, rad, lines, ld_lf, st_lf, b - 2048, fixed_nt, 0, pp, true, &f) <= 0) continue;
+            Mix r = shape(m, rev, f.lpw, f.nt, ld_lf, st_lf, true);
+            if (r.pp && !pp) continue;
+            f.lstr = r.lstr = std::max(f.lstr, r.lstr);
+            f.pp = r.pp = f.pp || r.pp ? f.lpw * f.lstr : 0;
+            out->f = f;
+            out->r = r;
+            if (mix_conv_lds_bytes(arith, *out) <= budget) return true;
+        }
+    return false;
+}
+
 }  // namespace mifft

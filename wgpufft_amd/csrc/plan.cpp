@@ -851,6 +851,33 @@ struct Builder {
         return false;
     }
 
+    // Schedule of a fused convolution of length m (op.conv.io set): the
+    // register form (mix_conv.hpp) for at least two stages, the LDS-to-LDS one
+    // for shorter lengths and given (medium prime) radices.  The schedule
+    // depends on m alone.
+    void conv_schedule(Op& op, uint64_t m, uint32_t lpw, bool ld_lf, bool st_lf, const std::vector<int>* radices) {
+        MixConv mc;
+        if (!radices && mix_conv_plan(P.arith, m, op.conv.io.lines, ld_lf, st_lf, P.lds_budget, P.batch_mode ? 256 : 0, &mc)) {
+            op.conv.mx = mc;
+            op.conv.mix = 1;
+            const std::vector<int> rad = mix_schedule(m);
+            op.conv.io.tw = stage_twiddles(P.arith, rad);
+            op.conv.mx.rtw = stage_twiddles(P.arith, std::vector<int>(rad.rbegin(), rad.rend()));
+            return;
+        }
+        op.conv.mix = 0;
+        op.conv.sc = make_sched(m, lpw, ld_lf, st_lf, radices);
+        op.conv.io.tw = stage_twiddles(P.arith, sched_radices(op.conv.sc));
+    }
+    static std::string conv_str(const Op& op, uint64_t m) {
+        return op.conv.mix ? radices_str(mix_schedule(m)) : sched_str(op.conv.sc);
+    }
+    static std::string conv_shape_str(const Op& op) {
+        if (!op.conv.mix) return " lpw=" + std::to_string(op.conv.sc.lpw);
+        return " lpw=" + std::to_string(op.conv.mx.f.lpw) + " nt=" + std::to_string(op.conv.mx.f.nt) +
+               (op.conv.mx.f.pp ? " pp" : "");
+    }
+
     void rader_op(uint64_t p, uint64_t m, uint32_t lpw, const LineSet& ls, const Layout& in,
                   const Layout& out, int src, uint64_t src_off, int dst, uint64_t dst_off,
                   bool conj_in, bool conj_out, double scale, const std::vector<int>* radices = nullptr) {
@@ -881,8 +908,7 @@ struct Builder {
         op.dst_off = dst_off;
         op.prec = P.prec;
         op.conv.io = base_args(ls, in, out, conj_in, conj_out, scale);
-        op.conv.sc = make_sched(m, lpw, adjacent_lines(ls, in), adjacent_lines(ls, out), radices);
-        op.conv.io.tw = stage_twiddles(P.arith, sched_radices(op.conv.sc));
+        conv_schedule(op, m, lpw, adjacent_lines(ls, in), adjacent_lines(ls, out), radices);
         op.conv.filt = filt;
         op.conv.perm_in = dpin;
         op.conv.perm_out = dpout;
@@ -890,8 +916,7 @@ struct Builder {
         op.conv.m = (uint32_t)m;
         op.conv.dn = make_magic((uint32_t)p);
         std::ostringstream d;
-        d << "rader p=" << p << " M=" << m << " " << sched_str(op.conv.sc) << " lines=" << ls.lines
-          << " lpw=" << lpw;
+        d << "rader p=" << p << " M=" << m << " " << conv_str(op, m) << " lines=" << ls.lines << conv_shape_str(op);
         op.desc = d.str();
         P.ops.push_back(op);
     }
@@ -923,15 +948,13 @@ struct Builder {
         op.dst_off = dst_off;
         op.prec = P.prec;
         op.conv.io = base_args(ls, in, out, conj_in, conj_out, scale);
-        op.conv.sc = make_sched(m, lpw, adjacent_lines(ls, in), adjacent_lines(ls, out));
-        op.conv.io.tw = stage_twiddles(P.arith, sched_radices(op.conv.sc));
+        conv_schedule(op, m, lpw, adjacent_lines(ls, in), adjacent_lines(ls, out), nullptr);
         op.conv.filt = bluestein_filter(n, m);
         op.conv.chirp = chirp_table(n);
         op.conv.n = (uint32_t)n;
         op.conv.m = (uint32_t)m;
         std::ostringstream d;
-        d << "bluestein N=" << n << " M=" << m << " " << sched_str(op.conv.sc)
-          << " lines=" << ls.lines << " lpw=" << lpw;
+        d << "bluestein N=" << n << " M=" << m << " " << conv_str(op, m) << " lines=" << ls.lines << conv_shape_str(op);
         op.desc = d.str();
         P.ops.push_back(op);
     }
@@ -1946,7 +1969,8 @@ static void run_op(const Op& op, hipStream_t s, const void* in, void* out, void*
             ConvArgs c = op.conv;
             c.io.in = ptr(op.src, op.src_off);
             c.io.out = ptr(op.dst, op.dst_off);
-            hip_check(op.kind == OP_RADER ? launch_rader(op.prec, c, s)
+            hip_check(c.mix                ? launch_mix_conv(op.prec, op.kind == OP_RADER, c, s)
+                      : op.kind == OP_RADER ? launch_rader(op.prec, c, s)
                       : op.rcv            ? launch_reg_bluestein(op.rcv, c, s)
                                           : launch_bluestein(op.prec, c, s),
                       "convolution kernel");
