@@ -5,7 +5,9 @@ namespace mifft {
 
 hipError_t launch_mix_real(bool c2r, const LineArgs& a, const Mix& mx, hipStream_t s) {
     if (mx.nt > 1024 || mx.ns < 2 || !mx.pairs) return hipErrorInvalidValue;
-    const void* fn = c2r ? (const void*)&mix_real_kernel<true> : (const void*)&mix_real_kernel<false>;
+    const void* fn = c2r         ? (const void*)&mix_real_kernel<true, false>
+                     : mx.stream ? (const void*)&mix_real_kernel<false, true>
+                                 : (const void*)&mix_real_kernel<false, false>;
     const size_t bytes = mix_lds_bytes(P_F32, mx);
     hipError_t e = ensure_lds_attr(fn, bytes);
     if (e != hipSuccess) return e;

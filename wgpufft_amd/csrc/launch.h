@@ -88,6 +88,7 @@ struct Mix {
     // k, n - k per line, n / 2 + 1 of them; 0 for complex lines
     uint32_t pairs, dpairs;
     MixStage st[kMixStages];
+    uint32_t stream;  // non-temporal loads of stage 0
 };
 std::vector<int> mix_schedule(uint64_t n);
 // Tile of `lines` lines of n points within `budget` bytes of LDS; fixed_nt /

@@ -307,8 +307,12 @@ __device__ __forceinline__ void mix_conv_tile(const ConvArgs& c, unsigned char* 
     }
 }
 
+// f64 tiles of up to 512 threads keep three waves per SIMD (168 registers; 198
+// unbounded leave two): 4096 lines of 1009 points 66 -> 58 us, Bluestein 611
+// points 74 -> 64.  In f32 a bound below the 111 registers asked for measured
+// slower.
 template <class Fmt, bool RADER, int NT>
-__global__ void __launch_bounds__(NT) mix_conv_kernel(ConvArgs c) {
+__global__ void __launch_bounds__(NT, Fmt::kId == 0 || NT > 512 ? 4 : 3) mix_conv_kernel(ConvArgs c) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     mix_conv_tile<Fmt, RADER>(c, smem_raw, xcd_remap(blockIdx.x, gridDim.x) * c.mx.f.lpw);
 }

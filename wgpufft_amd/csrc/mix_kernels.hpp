@@ -20,8 +20,13 @@
 // LDS-to-LDS engine, in us: 1000 x 4000 columns and rows (the passes of 10^6
 // points x 4) 87 -> 46; 270 x 28822 59 -> 36; one 1000-point line 12.4 -> 7.1
 // (call included); 104x140x60 f64 forward and inverse 118 -> 61.
-// Loads are plain ones: a butterfly's runs of n / R points share cache lines
-// with their neighbours'.
+//
+// Loads are non-temporal (mx.stream; kernels of their own) where a pass reads 32 MiB or more in runs
+// of at least 192 bytes, or strided rows of 128 (64 MiB in and out: 1000
+// points 39.4 -> 32.8 us, 1920 36.1 -> 31.4, 60-point rows 31.1 -> 27.6).
+// Shorter runs share cache lines with their neighbours' (60 contiguous points
+// 36.3 -> 41.5 us with the hint, 32-byte strided rows 45.6 -> 53.2), and
+// smaller arrays stay in the last-level cache (3-8 % slower with it).
 //
 // LDS layout between stage s (radix R, previous product L) and the next: output
 // m of butterfly j at m * nrp + j, nrp = (n / R) | 1.  Writes are contiguous
@@ -98,7 +103,7 @@ __device__ __forceinline__ void mix_put(const Mix& mx, const MixStage& st, cpx<T
 
 // Stage 0: memory -> LDS.  Lines past the end read the last line and are
 // never stored.
-template <class Fmt, int LDM, int R, int NB>
+template <class Fmt, int LDM, bool NTL, int R, int NB>
 __device__ __forceinline__ void mix_first(const LineArgs& a, const Mix& mx, cpx<typename Fmt::T>* dst, uint32_t g0) {
     using T = typename Fmt::T;
     const MixStage& st = mx.st[0];
@@ -114,7 +119,7 @@ __device__ __forceinline__ void mix_first(const LineArgs& a, const Mix& mx, cpx<
             const LineBase lb = line_base(a, g < a.lines ? g : a.lines - 1);
             const uint32_t o0 = lb.in + at[q].j * (uint32_t)a.in_sn, sn = st.nr * (uint32_t)a.in_sn;
 #pragma unroll
-            for (int i = 0; i < R; i++) w[q][i] = load_point_at<Fmt, LDM, false>(a, o0 + i * sn);
+            for (int i = 0; i < R; i++) w[q][i] = load_point_at<Fmt, LDM, NTL>(a, o0 + i * sn);
         }
 #pragma unroll
         for (int q = 0; q < NB; q++) {
@@ -180,19 +185,25 @@ __device__ __forceinline__ void mix_last(const LineArgs& a, const Mix& mx, const
     }
 }
 
-// Lines [g0, g0 + lpw) of ns >= 2 stages: memory -> stages -> memory.
-template <class Fmt, int LDM, int STM, bool POST>
-__device__ __forceinline__ void mix_tile(const LineArgs& a, const Mix& mx, unsigned char* smem, uint32_t g0) {
-    using T = typename Fmt::T;
-    cpx<T>* src = reinterpret_cast<cpx<T>*>(smem);
-    cpx<T>* dst = src + mx.pp;
+template <class Fmt, int LDM, bool NTL>
+__device__ __forceinline__ void mix_load(const LineArgs& a, const Mix& mx, cpx<typename Fmt::T>* dst, uint32_t g0) {
     switch (mx.st[0].code) {
 #define MIFFT_MIX_CASE(R, NB) \
-    case R + 32 * NB: mix_first<Fmt, LDM, R, NB>(a, mx, src, g0); break;
+    case R + 32 * NB: mix_first<Fmt, LDM, NTL, R, NB>(a, mx, dst, g0); break;
         MIFFT_MIX_RADICES(MIFFT_MIX_CASE)
 #undef MIFFT_MIX_CASE
         default: break;
     }
+}
+
+// Lines [g0, g0 + lpw) of ns >= 2 stages: memory -> stages -> memory.
+// NTL: non-temporal loads.
+template <class Fmt, int LDM, int STM, bool POST, bool NTL = false>
+__device__ __forceinline__ void mix_tile(const LineArgs& a, const Mix& mx, unsigned char* smem, uint32_t g0) {
+    using T = typename Fmt::T;
+    cpx<T>* src = reinterpret_cast<cpx<T>*>(smem);
+    cpx<T>* dst = src + mx.pp;
+    mix_load<Fmt, LDM, NTL>(a, mx, src, g0);
     __syncthreads();
 #pragma nounroll
     for (uint32_t s = 1; s + 1 < mx.ns; s++) {
@@ -330,7 +341,7 @@ __device__ __forceinline__ void mix_pairs_in(const LineArgs& a, const Mix& mx, c
 }
 
 // Lines [g0, g0 + lpw) of 2n real points (a's real side in complex elements).
-template <bool C2R>
+template <bool C2R, bool NTL = false>
 __device__ __forceinline__ void mix_real_tile(const LineArgs& a, const Mix& mx, unsigned char* smem, uint32_t g0) {
     using T = float;
     cpx<T>* src = reinterpret_cast<cpx<T>*>(smem);
@@ -350,13 +361,7 @@ __device__ __forceinline__ void mix_real_tile(const LineArgs& a, const Mix& mx, 
         src = dst;
         dst = x;
     } else {
-        switch (mx.st[0].code) {
-#define MIFFT_MIX_CASE(R, NB) \
-    case R + 32 * NB: mix_first<FmtF32, LD_COMPLEX, R, NB>(a, mx, src, g0); break;
-            MIFFT_MIX_RADICES(MIFFT_MIX_CASE)
-#undef MIFFT_MIX_CASE
-            default: break;
-        }
+        mix_load<FmtF32, LD_COMPLEX, NTL>(a, mx, src, g0);
     }
     __syncthreads();
 #pragma nounroll
@@ -396,17 +401,18 @@ __device__ __forceinline__ void mix_real_tile(const LineArgs& a, const Mix& mx, 
     }
 }
 
-template <bool C2R>
+template <bool C2R, bool NTL>
 __global__ void __launch_bounds__(1024) mix_real_kernel(LineArgs a, Mix mx) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    mix_real_tile<C2R>(a, mx, smem_raw, xcd_remap(blockIdx.x, gridDim.x) * mx.lpw);
+    mix_real_tile<C2R, NTL>(a, mx, smem_raw, xcd_remap(blockIdx.x, gridDim.x) * mx.lpw);
 }
 
-// NT: the launch bound (the register budget).
-template <class Fmt, int LDM, int STM, bool POST, int NT>
+// NT: the launch bound.  Register budgets below what the stages ask for (72 or
+// 64 in f32, 128 for 512 threads in f64) spill and measured 5-15 % slower.
+template <class Fmt, int LDM, int STM, bool POST, int NT, bool NTL>
 __global__ void __launch_bounds__(NT) mix_fft_kernel(LineArgs a, Mix mx) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    mix_tile<Fmt, LDM, STM, POST>(a, mx, smem_raw, xcd_remap(blockIdx.x, gridDim.x) * mx.lpw);
+    mix_tile<Fmt, LDM, STM, POST, NTL>(a, mx, smem_raw, xcd_remap(blockIdx.x, gridDim.x) * mx.lpw);
 }
 
 }  // namespace mifft

@@ -216,7 +216,11 @@ bool mix_plan(int arith, uint64_t n, uint64_t lines, bool ld_lf, bool st_lf, siz
     // (several rounds per middle stage) only where nothing else does
     for (int pp = 0; pp < 2; pp++)
         for (size_t b : {fixed_nt ? budget / 2 : budget, budget})
-            if (best_shape(arith, n, rad, lines, ld_lf, st_lf, b, fixed_nt, forced_lpw, pp, real, out) > 0) return true;
+            if (best_shape(arith, n, rad, lines, ld_lf, st_lf, b, fixed_nt, forced_lpw, pp, real, out) > 0) {
+                const uint64_t es = arith == P_F32 ? 8 : 16;
+                out->stream = lines * n * es >= (32u << 20) && (ld_lf ? out->lpw * es >= 128 : out->st[0].nr * es >= 192);
+                return true;
+            }
     return false;
 }
 
