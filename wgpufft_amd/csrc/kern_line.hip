@@ -272,17 +272,22 @@ static const RegVariant kRegistry[] = {
     REGP(FmtF32, P_F32, 2048, 128, 2, 0, 0, LD_REAL, ST_PACKED, 0, 1, 2, "16x16x8", 16, 16, 8),
     REGP(FmtF32, P_F32, 2048, 128, 1, 0, 0, LD_HERMITIAN, ST_REAL, 0, 1, 2, "16x16x8", 16, 16, 8),
     REGP(FmtF32, P_F32, 2048, 128, 2, 0, 0, LD_HERMITIAN, ST_REAL, 0, 1, 2, "16x16x8", 16, 16, 8),
-    // fold passes of 2D transforms (rows r + c M/F of the second axis per thread)
+    // fold passes of 2D transforms (rows r + c M/F of the second axis per
+    // thread); the defaults hold 8 points per thread and line, which leaves
+    // registers for twice the waves of the 16-point forms (one transform:
+    // 4096 x 2048 61.0 -> 56.8 us with 16-byte accesses as well, 2048^2 32.0
+    // -> 31.2, 1024^2 17.3 -> 16.5)
+    REGFA(4096, 256, 2, "8x8x8x8", 8, 8, 8, 8),
     REGF(FmtF32, P_F32, 4096, 256, 2, "16x16x16", 16, 16, 16),
     REGF(FmtF32, P_F32, 4096, 512, 2, "8x8x8x8", 8, 8, 8, 8),
     REGFP(FmtF32, P_F32, 4096, 512, 2, 1, "8x8x8x8", 8, 8, 8, 8),
     REGFP(FmtF32, P_F32, 4096, 512, 2, 2, "8x8x8x8", 8, 8, 8, 8),
     REGFP(FmtF32, P_F32, 4096, 256, 2, 1, "16x16x16", 16, 16, 16),
     REGF(FmtF32, P_F32, 4096, 512, 4, "8x8x8x8", 8, 8, 8, 8),
-    REGF(FmtF32, P_F32, 2048, 128, 2, "16x16x8", 16, 16, 8),
     REGF(FmtF32, P_F32, 2048, 256, 2, "8x8x8x4", 8, 8, 8, 4),
-    REGF(FmtF32, P_F32, 1024, 64, 2, "16x16x4", 16, 16, 4),
+    REGF(FmtF32, P_F32, 2048, 128, 2, "16x16x8", 16, 16, 8),
     REGF(FmtF32, P_F32, 1024, 128, 2, "8x8x4x4", 8, 8, 4, 4),
+    REGF(FmtF32, P_F32, 1024, 64, 2, "16x16x4", 16, 16, 4),
     // R2C fold: real rows r, r + M/2 in, packed rows out
     REGFM(FmtF32, P_F32, 2048, 128, 2, LD_REAL, ST_PACKED, "16x16x8", 16, 16, 8),
     REGFM(FmtF32, P_F32, 2048, 256, 2, LD_REAL, ST_PACKED, "8x8x8x4", 8, 8, 8, 4),
@@ -291,9 +296,14 @@ static const RegVariant kRegistry[] = {
     REGFM(FmtF32, P_F32, 2048, 256, 2, LD_HERMITIAN, ST_REAL, "8x8x8x4", 8, 8, 8, 4),
     REGFM(FmtF32, P_F32, 1024, 64, 2, LD_REAL, ST_PACKED, "16x16x4", 16, 16, 4),
     REGFM(FmtF32, P_F32, 1024, 64, 2, LD_HERMITIAN, ST_REAL, "16x16x4", 16, 16, 4),
-    // smaller tiles: more tiles per persistent workgroup, a shorter pipeline tail
+    // smaller tiles: more tiles per persistent workgroup, a shorter pipeline
+    // tail; the default of long batches (4096 x 2048 points 32.0 -> 25.8 us,
+    // 8192 x 512 16.2 -> 14.6, 32768 x 256 26.5 -> 24.2; 128-point lines lose
+    // 2-20 %, strided columns 2-18 %)
     REGP(FmtF32, P_F32, 1024, 64, 2, 0, 0, LD_COMPLEX, ST_COMPLEX, 0, 1, 2, "16x16x4", 16, 16, 4),
-    REGP(FmtF32, P_F32, 1024, 128, 2, 0, 0, LD_COMPLEX, ST_COMPLEX, 0, 1, 2, "8x8x4x4", 8, 8, 4, 4),
+    REGP(FmtF32, P_F32, 2048, 128, 1, 0, 0, LD_COMPLEX, ST_COMPLEX, 0, 1, 2, "16x16x8", 16, 16, 8),
+    REGP(FmtF32, P_F32, 512, 32, 4, 0, 0, LD_COMPLEX, ST_COMPLEX, 0, 1, 2, "8x8x8", 8, 8, 8),
+    REGP(FmtF32, P_F32, 256, 16, 8, 0, 0, LD_COMPLEX, ST_COMPLEX, 0, 1, 2, "16x16", 16, 16),
     // persistent pipelined form of the first pass of a 2^20-point split
     // (16384 lines of 64 points; with two tiles per workgroup the next tile's
     // loads overlap the current tile's stages and stores: 41.3 vs 43.3 us per
@@ -304,7 +314,6 @@ static const RegVariant kRegistry[] = {
     REGV(FmtF64, P_F64, 4096, 128, 4, 1, 1, LD_COMPLEX, ST_COMPLEX, 1, 1, "16x16x16", 16, 16, 16),
     REGV(FmtF64, P_F64, 4096, 128, 4, 0, 1, LD_COMPLEX, ST_COMPLEX, 0, 1, "16x16x16", 16, 16, 16),
     // adjacent-butterfly forms: 16-byte loads and stores of contiguous lines
-    REGFA(4096, 256, 2, "8x8x8x8", 8, 8, 8, 8),
     REGFA(4096, 256, 2, "8x16x8x4", 8, 16, 8, 4),
     REGFA(4096, 128, 2, "8x8x8x8", 8, 8, 8, 8),
     REGFA(4096, 128, 2, "16x16x16", 16, 16, 16),

@@ -626,25 +626,95 @@ struct Builder {
         return a;
     }
 
-    // Few lines: the default shape of a pass (the first registered variant,
-    // measured on arrays of 64 MiB and more) can leave most CUs idle (2048
-    // lines of 512 points in 64 workgroups); then the variant of the same
-    // shape and radix schedule with the most workgroups, up to two per CU,
-    // runs instead.  The schedule fixes a line's arithmetic, so a line's
-    // result does not depend on how many lines its plan has.
-    const RegVariant* filling_variant(const RegVariant* rv, uint64_t n, uint64_t lines, bool ld_lf, bool st_lf,
-                                      int ldm, int stm, int post, bool pairable) {
-        const uint64_t want = 2ull * device_cu_count();
-        auto wgs = [&](const RegVariant* v) { return std::min<uint64_t>(want, (lines + v->lines - 1) / v->lines); };
-        if (wgs(rv) >= want) return rv;
-        const RegVariant* best = rv;
-        for (const RegVariant* v : find_reg_variants(P.prec, (int)n, ld_lf, st_lf, ldm, stm, post)) {
-            if (v->adj || v->persist || v->fold || (v->vec == 2 && !pairable) || v->lds_bytes > P.lds_budget ||
-                std::strcmp(v->radices, rv->radices) != 0)
-                continue;
-            if (wgs(v) > wgs(best)) best = v;
-        }
+    // The variant of rv's length, layout and radix schedule that runs `lines`
+    // lines fastest (rv: the first registered one).  The schedule fixes a
+    // line's arithmetic, so a line's result does not depend on how many lines
+    // its plan has.
+    const RegVariant* sized_variant(const RegVariant* rv, uint64_t n, uint64_t lines, bool ld_lf, bool st_lf,
+                                    int ldm, int stm, int post, bool pairable) {
+        std::vector<const RegVariant*> same;
+        for (const RegVariant* v : find_reg_variants(P.prec, (int)n, ld_lf, st_lf, ldm, stm, post))
+            if (!v->adj && !v->fold && (v->vec == 1 || pairable) && v->lds_bytes <= P.lds_budget &&
+                std::strcmp(v->radices, rv->radices) == 0)
+                same.push_back(v);
+        const uint64_t cus = device_cu_count();
+        auto tiles = [&](const RegVariant* v) { return (lines + v->lines - 1) / v->lines; };
+        if (P.prec == P_F32 && ldm == LD_COMPLEX && stm == ST_COMPLEX && (ld_lf || st_lf))
+            return strided_variant(rv, same, n, lines, ld_lf, post);
+        // Contiguous complex lines with at least eight tiles per CU: the
+        // persistent pipelined form of the smallest tile, whose loads of the
+        // next tile run under the stages of the current one.  4096 x 1024
+        // points 12.2 -> 10.5 us, 16384 x 1024 63 -> 51, 2048 x 4096 20.9 ->
+        // 18.9, 4096 x 4096 62 -> 52, 16384 x 4096 (beyond the last-level
+        // cache, both forms wait for HBM) 204 -> 203; with four tiles per CU
+        // 1024 x 4096 10.9 -> 11.3, 2048 x 1024 no better than two lines per
+        // workgroup.
+        const RegVariant* best = nullptr;
+        if (ldm == LD_COMPLEX && stm == ST_COMPLEX)
+            for (const RegVariant* v : same)
+                if (v->persist && tiles(v) >= 8 * cus && (!best || v->lines < best->lines)) best = v;
+        if (best) return best;
+        // Few lines: the first registered shape (measured on arrays of 64 MiB
+        // and more) can leave most CUs idle; then the shape with the most
+        // workgroups, up to four per CU (2048 x 1024 points at 512 and 1024
+        // workgroups: 7.6 and 7.0 us).
+        const uint64_t want = 4 * cus;
+        auto wgs = [&](const RegVariant* v) { return std::min(want, tiles(v)); };
+        best = rv;
+        for (const RegVariant* v : same)
+            if (!v->persist && wgs(v) > wgs(best)) best = v;
         return best;
+    }
+
+    // Strided f32 lines (lines-fastest loads, stores or both).  A workgroup of
+    // `want` lines reads or writes rows of 8 want bytes; more lines give
+    // longer rows, fewer more workgroups (and LDS for more of them per CU).
+    // While the arrays sit in the last-level cache 64-byte rows are enough
+    // and the smaller tiles win: 8 lines per workgroup for 256 points and up
+    // (8160 columns of 512 points 27.6 us against 30.4 at 32 and 4;  4128 of
+    // 1024 points, in pairs, 30.6 against 34.2 one by one; 2016 of 2048 31.4
+    // against 39.1 at 2; 8192 of a 4096 x 2048 fold 16 us less than 16 lines
+    // one by one), 32 for shorter lines, 8 for 128-point lines that store
+    // with a twiddle (32768 of them 27.3 against 28.4 at 32), and
+    // min(16, 4096 / n) for contiguous loads with transposed stores (16384
+    // of 512 points 51.5 against 53.4 at 16; 8192 of 1024 59.8 against 61.4).
+    // Arrays beyond the cache want 128-byte rows and more: the first
+    // registered shape, but 16 lines at 512 and 1024 points in pairs (1024
+    // points, 128 MiB: 111 us against 130 at 32), and 8 lines at 2048 (64
+    // MiB: 67 against 77 at 16, 256 MiB: equal).  The line between them, per
+    // array: 48 MiB below 1024 points (256-point columns of 64 MiB: 58.1 us
+    // at 8 lines, 55.7 at 32), 96 MiB from there up and for transposed
+    // stores of 512 points (1024-point columns of 64 MiB: 58.1 at 8, 59.8 at
+    // 16; 512-point rows of 128 MiB: equal).  Short of a workgroup for every
+    // second CU the tile halves until that is reached (288 columns of 1024
+    // points: 12.3, 11.5 and 11.1 us at 8, 4 and 2; 1056 columns are faster
+    // at 8 than at 4).
+    const RegVariant* strided_variant(const RegVariant* rv, const std::vector<const RegVariant*>& same, uint64_t n,
+                                      uint64_t lines, bool ld_lf, int post) {
+        const bool columns = ld_lf && !post;
+        const uint64_t points = n * lines;
+        const uint64_t cache_points = n >= 1024 || (!ld_lf && n == 512) ? 12u << 20 : 6u << 20;
+        uint64_t want;
+        if (points >= cache_points) {
+            if (!columns || n < 512 || n > 2048) return rv;
+            want = n == 2048 ? 8 : 16;
+            if (rv->vec != 2) return rv;
+        } else if (!ld_lf) {
+            want = std::min<uint64_t>(16, std::max<uint64_t>(1, 4096 / n));
+        } else {
+            want = n >= 256 || (post && n == 128) ? 8 : 32;
+        }
+        while (want > 1 && 2 * ((lines + want - 1) / want) < device_cu_count()) want /= 2;
+        // the widest shape of at most `want` lines, pairs first; else the narrowest
+        const RegVariant *best = nullptr, *narrow = nullptr;
+        for (const RegVariant* v : same) {
+            if (v->persist) continue;
+            if (v->lines <= (int)want &&
+                (!best || v->lines > best->lines || (v->lines == best->lines && v->vec > best->vec)))
+                best = v;
+            if (!narrow || v->lines < narrow->lines) narrow = v;
+        }
+        return best ? best : narrow ? narrow : rv;
     }
 
     // Line stride of the real side of a contiguous real line op: n real
@@ -768,7 +838,7 @@ struct Builder {
         } else if (!tuned) {
             rv = pairable ? find_reg_variant(P.prec, (int)n, ld_lf, st_lf, ldm, stm, post, 2) : nullptr;
             if (!rv) rv = find_reg_variant(P.prec, (int)n, ld_lf, st_lf, ldm, stm, post, 1);
-            if (rv) rv = filling_variant(rv, n, ls.lines, ld_lf, st_lf, ldm, stm, post, pairable);
+            if (rv) rv = sized_variant(rv, n, ls.lines, ld_lf, st_lf, ldm, stm, post, pairable);
         }
         const size_t es = elem_bytes(P.arith);
         const uint64_t lstr = lds_line_stride((uint32_t)std::min<uint64_t>(n, 1u << 30));
@@ -1344,8 +1414,14 @@ struct Builder {
                     fold_in % 2 == 0 && fold_out % 2 == 0;
         const RegVariant* rv = find_reg_variant_named(tuning_lookup(op.tkey));
         if (!rv || rv->fold != (int)F || rv->n != (int)n0 || rv->prec != P.prec || rv->ldm != ldm ||
-            rv->stm != stm || (rv->adj && !op.adj_ok))
-            rv = fv[0];
+            rv->stm != stm || (rv->adj && !op.adj_ok)) {
+            rv = nullptr;
+            for (const RegVariant* v : fv)
+                if (!v->adj || op.adj_ok) {
+                    rv = v;
+                    break;
+                }
+        }
         op.rv = rv;
         op.a = base_args(ls, lay_in, lay_out, conj, conj, scale);
         op.a.fold_in = (uint32_t)fold_in;
