@@ -69,3 +69,34 @@ def test_column_counts_agree(n):
             assert np.linalg.norm(got - ref) <= 6e-7 * np.linalg.norm(ref)
         else:
             assert torch.equal(y[:, :2], base[1]), (n, w)
+
+
+# real lines below and above the persistent form's eight tiles per CU
+@pytest.mark.parametrize("kind,n,counts", [
+    ("r2c", 256, (8189, 8195)), ("r2c", 512, (8189, 8195)),
+    ("r2c", 1024, (4093, 4099)), ("r2c", 2048, (2047, 2049)), ("r2c", 4096, (2047, 2049)),
+    ("c2r", 1024, (4093, 4099)), ("c2r", 2048, (2047, 2049)), ("c2r", 4096, (2047, 2049)),
+    ("c2r", 64, (5, 4099)), ("c2r", 512, (3, 2049))])
+def test_real_counts_agree(kind, n, counts):
+    pin, pout = (n, n + 2) if kind == "r2c" else (n + 2, n)  # floats per line
+    x = uniform(pin * max(counts) // 2 + 1, n)[:pin * max(counts)].view(-1, pin)
+    if kind == "c2r":  # Hermitian: real first and last bins
+        x[:, 1] = 0
+        x[:, n + 1] = 0
+    outs = []
+    for c in counts:
+        cfg = (FftConfig.new(n) if kind == "r2c" else FftConfig.inverse(n)).with_batch(c)
+        plan = getattr(FftPlan, kind)(cfg)
+        y = torch.empty(c * pout, device="cuda")
+        plan.execute(x[:c].contiguous(), y)
+        torch.cuda.synchronize()
+        outs.append(y.view(c, pout))
+    m = min(counts)
+    assert torch.equal(outs[0][:m], outs[1][:m])
+    xs = x[:3].cpu().numpy().astype(np.float64)
+    if kind == "r2c":
+        ref = np.fft.rfft(xs).view(np.float64).reshape(3, pout)
+    else:
+        ref = np.fft.irfft(xs.view(np.complex128), n)
+    got = outs[0][:3].cpu().numpy()
+    assert np.linalg.norm(got - ref) <= 6e-7 * np.linalg.norm(ref)

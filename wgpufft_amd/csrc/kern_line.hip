@@ -267,11 +267,17 @@ static const RegVariant kRegistry[] = {
     // persistent pipelined forms of the strided column-pair passes of 2D
     // folds (1024-point columns of a 4096 x 2048 fold)
     REGP(FmtF32, P_F32, 1024, 128, 8, 1, 1, LD_COMPLEX, ST_COMPLEX, 0, 2, 2, "8x8x4x4", 8, 8, 4, 4),
-    // persistent pipelined forms of the 2048^2 real passes (axis 0)
+    // persistent pipelined forms of the real passes (axis 0)
     REGP(FmtF32, P_F32, 2048, 128, 1, 0, 0, LD_REAL, ST_PACKED, 0, 1, 2, "16x16x8", 16, 16, 8),
     REGP(FmtF32, P_F32, 2048, 128, 2, 0, 0, LD_REAL, ST_PACKED, 0, 1, 2, "16x16x8", 16, 16, 8),
     REGP(FmtF32, P_F32, 2048, 128, 1, 0, 0, LD_HERMITIAN, ST_REAL, 0, 1, 2, "16x16x8", 16, 16, 8),
     REGP(FmtF32, P_F32, 2048, 128, 2, 0, 0, LD_HERMITIAN, ST_REAL, 0, 1, 2, "16x16x8", 16, 16, 8),
+    REGP(FmtF32, P_F32, 4096, 256, 1, 0, 0, LD_REAL, ST_PACKED, 0, 1, 2, "16x16x16", 16, 16, 16),
+    REGP(FmtF32, P_F32, 1024, 64, 2, 0, 0, LD_REAL, ST_PACKED, 0, 1, 2, "16x16x4", 16, 16, 4),
+    REGP(FmtF32, P_F32, 512, 32, 4, 0, 0, LD_REAL, ST_PACKED, 0, 1, 1, "8x8x8", 8, 8, 8),
+    REGP(FmtF32, P_F32, 256, 16, 4, 0, 0, LD_REAL, ST_PACKED, 0, 1, 1, "16x16", 16, 16),
+    REGP(FmtF32, P_F32, 4096, 256, 1, 0, 0, LD_HERMITIAN, ST_REAL, 0, 1, 2, "16x16x16", 16, 16, 16),
+    REGP(FmtF32, P_F32, 1024, 64, 2, 0, 0, LD_HERMITIAN, ST_REAL, 0, 1, 2, "16x16x4", 16, 16, 4),
     // fold passes of 2D transforms (rows r + c M/F of the second axis per
     // thread); the defaults hold 8 points per thread and line, which leaves
     // registers for twice the waves of the 16-point forms (one transform:

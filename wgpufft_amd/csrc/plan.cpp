@@ -641,7 +641,7 @@ struct Builder {
         auto tiles = [&](const RegVariant* v) { return (lines + v->lines - 1) / v->lines; };
         if (P.prec == P_F32 && ldm == LD_COMPLEX && stm == ST_COMPLEX && (ld_lf || st_lf))
             return strided_variant(rv, same, n, lines, ld_lf, post);
-        // Contiguous complex lines with at least eight tiles per CU: the
+        // Contiguous lines with at least eight tiles per CU: the
         // persistent pipelined form of the smallest tile, whose loads of the
         // next tile run under the stages of the current one.  4096 x 1024
         // points 12.2 -> 10.5 us, 16384 x 1024 63 -> 51, 2048 x 4096 20.9 ->
@@ -649,8 +649,10 @@ struct Builder {
         // cache, both forms wait for HBM) 204 -> 203; with four tiles per CU
         // 1024 x 4096 10.9 -> 11.3, 2048 x 1024 no better than two lines per
         // workgroup.
+        // Real lines gain the same way (R2C of 8192 x 1024 points 18.0 ->
+        // 15.2, of 8192 x 2048 39.4 -> 28.5; C2R 22.5 -> 19.5 and 42.1 -> 33.1).
         const RegVariant* best = nullptr;
-        if (ldm == LD_COMPLEX && stm == ST_COMPLEX)
+        if (P.prec == P_F32)
             for (const RegVariant* v : same)
                 if (v->persist && tiles(v) >= 8 * cus && (!best || v->lines < best->lines)) best = v;
         if (best) return best;
@@ -677,15 +679,17 @@ struct Builder {
     // one by one), 32 for shorter lines, 8 for 128-point lines that store
     // with a twiddle (32768 of them 27.3 against 28.4 at 32), and
     // min(16, 4096 / n) for contiguous loads with transposed stores (16384
-    // of 512 points 51.5 against 53.4 at 16; 8192 of 1024 59.8 against 61.4).
+    // of 512 points 51.5 against 53.4 at 16; 8192 of 1024 59.8 against 61.4;
+    // 32 at 64 points: 65536 of them 43.8 against 45.4 at 16).
     // Arrays beyond the cache want 128-byte rows and more: the first
     // registered shape, but 16 lines at 512 and 1024 points in pairs (1024
     // points, 128 MiB: 111 us against 130 at 32), and 8 lines at 2048 (64
     // MiB: 67 against 77 at 16, 256 MiB: equal).  The line between them, per
-    // array: 48 MiB below 1024 points (256-point columns of 64 MiB: 58.1 us
-    // at 8 lines, 55.7 at 32), 96 MiB from there up and for transposed
-    // stores of 512 points (1024-point columns of 64 MiB: 58.1 at 8, 59.8 at
-    // 16; 512-point rows of 128 MiB: equal).  Short of a workgroup for every
+    // array: 48 MiB (256-point columns of 64 MiB: 58.1 us at 8 lines, 55.7 at
+    // 32; 1024-point ones that store with a twiddle 75 against 66 at 16), 96
+    // MiB for plain columns of 1024 points and up and transposed stores of
+    // 512 and up (1024-point columns of 64 MiB: 58.1 at 8, 59.8 at 16;
+    // 512-point rows of 128 MiB: equal).  Short of a workgroup for every
     // second CU the tile halves until that is reached (288 columns of 1024
     // points: 12.3, 11.5 and 11.1 us at 8, 4 and 2; 1056 columns are faster
     // at 8 than at 4).
@@ -693,14 +697,14 @@ struct Builder {
                                       uint64_t lines, bool ld_lf, int post) {
         const bool columns = ld_lf && !post;
         const uint64_t points = n * lines;
-        const uint64_t cache_points = n >= 1024 || (!ld_lf && n == 512) ? 12u << 20 : 6u << 20;
+        const uint64_t cache_points = (columns && n >= 1024) || (!ld_lf && n >= 512) ? 12u << 20 : 6u << 20;
         uint64_t want;
         if (points >= cache_points) {
             if (!columns || n < 512 || n > 2048) return rv;
             want = n == 2048 ? 8 : 16;
             if (rv->vec != 2) return rv;
         } else if (!ld_lf) {
-            want = std::min<uint64_t>(16, std::max<uint64_t>(1, 4096 / n));
+            want = n < 128 ? 32 : std::min<uint64_t>(16, std::max<uint64_t>(1, 4096 / n));
         } else {
             want = n >= 256 || (post && n == 128) ? 8 : 32;
         }
@@ -840,6 +844,13 @@ struct Builder {
             if (!rv) rv = find_reg_variant(P.prec, (int)n, ld_lf, st_lf, ldm, stm, post, 1);
             if (rv) rv = sized_variant(rv, n, ls.lines, ld_lf, st_lf, ldm, stm, post, pairable);
         }
+        // C2R lines of up to 512 points run at half length (runtime_schedule):
+        // the register kernel reads every packed point twice and transforms
+        // the full length (131072 x 64 points 34.9 against 16.6 us, 32768 x
+        // 256 22.2 against 15.2, 16384 x 512 22.6 against 15.0, few lines
+        // equal; from 1024 points few lines are faster in the register
+        // kernel, 2048 x 1024 7.4 against 9.2 us at 2048 points)
+        if (!tuned && ldm == LD_HERMITIAN && n <= 512 && ls.S1 == 1 && ls.S2 == 1) rv = nullptr;
         const size_t es = elem_bytes(P.arith);
         const uint64_t lstr = lds_line_stride((uint32_t)std::min<uint64_t>(n, 1u << 30));
         if (rv && P.batch_mode && batch_class_for(rv) < 0) rv = nullptr;
