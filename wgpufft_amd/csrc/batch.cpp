@@ -337,10 +337,10 @@ uint32_t batch_grid(size_t lds_bytes) {
 
 void batch_enqueue(const BatchTile* const* d_tiles, const uint32_t* counts, const OpDesc* d_ops,
                    uint32_t* d_counters, uint32_t grid, size_t lds_bytes, hipStream_t s) {
-    hip_check(launch_batch_reset(d_counters, kMaxPhases, s), "batch reset");
+    hip_check(launch_batch_reset(d_counters, s), "batch reset");
     for (int k = 0; k < kMaxPhases; k++)
         if (counts[k])
-            hip_check(launch_batch(d_tiles[k], counts[k], d_counters + k, d_ops, std::min(grid, counts[k]),
+            hip_check(launch_batch(d_tiles[k], counts[k], d_counters, (uint32_t)k, d_ops, std::min(grid, counts[k]),
                                    lds_bytes, s),
                       "batch");
 }
@@ -407,7 +407,7 @@ static void create_batch(mifft_batch& B, const mifft_batch_item* items, int32_t 
     for (int k = 0; k < kMaxPhases; k++)
         upload((void**)&B.d_tiles[k], B.build.tiles[k].data(), B.build.tiles[k].size() * sizeof(BatchTile),
                "batch tiles");
-    hip_check(hipMalloc(&B.d_counters, 64), "batch counters");
+    hip_check(hipMalloc(&B.d_counters, kBatchCounterBytes), "batch counters");
 }
 
 static void run_batch(const mifft_batch& B, hipStream_t s) {

@@ -78,6 +78,11 @@ enum BatchClass : uint32_t {
 // launch each); ND transforms, four-step splits and multi-pass Bluestein
 // (chirp, padded FFT, filter, padded FFT, chirp) need more than one.
 constexpr int kMaxPhases = 8;
+// Tile counters of a phase, 64 bytes (kBatchQueueStride words) apart, and the
+// bytes that the counters of every phase take.
+constexpr uint32_t kBatchQueues = 8;
+constexpr uint32_t kBatchQueueStride = 16;
+constexpr size_t kBatchCounterBytes = (size_t)kMaxPhases * kBatchQueues * kBatchQueueStride * sizeof(uint32_t);
 // Elements per tile of the element-wise classes (16 per thread).
 constexpr uint32_t kEltTile = 4096;
 
@@ -103,8 +108,8 @@ int batch_class_for(const RegVariant* v);
 // store, register form), or -1.
 int batch_lds_class(int prec, int ldm, int stm, int post, bool mix);
 
-hipError_t launch_batch(const BatchTile* tiles, uint32_t ntiles, uint32_t* counter, const OpDesc* ops,
-                        uint32_t grid, size_t lds_bytes, hipStream_t s);
-hipError_t launch_batch_reset(uint32_t* counters, uint32_t n, hipStream_t s);
+hipError_t launch_batch(const BatchTile* tiles, uint32_t ntiles, uint32_t* counters, uint32_t phase,
+                        const OpDesc* ops, uint32_t grid, size_t lds_bytes, hipStream_t s);
+hipError_t launch_batch_reset(uint32_t* counters, hipStream_t s);
 
 }  // namespace mifft

@@ -20,15 +20,33 @@
 
 namespace mifft {
 
-// The tile claimed by the workgroup, broadcast through LDS.
-__shared__ uint32_t s_tile;
+// The tiles of a launch are dealt to kBatchQueues counters in runs of
+// neighbours (2^shift of them, run r to queue r mod kBatchQueues), workgroup b
+// claims from queue b mod kBatchQueues.  Workgroups b, b + 8, ... share an
+// XCD: neighbouring tiles of a pass then meet in one L2, which joins the
+// 128-byte lines that both touch (transforms start at any 16 bytes).  And
+// device atomics on one address are served one at a time, some 6 ns each.
+// Tiles are sorted by cost, so the queues hold equal work.  One counter and no
+// runs against this, by itself: 2047 transforms of 65536 points 1236 -> 1121
+// us, 2329 of 4096 63 -> 56, 2172 of 1001 40 -> 31, 2485 of 343 22 -> 15.
+// (Claiming the next tile before the current one's loads, to hide the atomic,
+// measured 1221: the in-order memory counter makes the loads wait for it.)
+//
+// The claimed index goes through s_next[0] and s_next[1] in turn, so that one
+// barrier per tile is enough (the one written was last read before the
+// previous barrier); bit 31 of a tile index says which of them the next claim
+// takes.
+__shared__ uint32_t s_next[2];
+constexpr uint32_t kSlotBit = 0x80000000u;
 
-__device__ __forceinline__ uint32_t claim_tile(uint32_t* counter) {
-    if (threadIdx.x == 0) s_tile = atomicAdd(counter, 1u);
-    __syncthreads();
-    const uint32_t t = __builtin_amdgcn_readfirstlane(s_tile);
-    __syncthreads();  // the next claim overwrites s_tile
-    return t;
+// queues: this workgroup's queue q, the number of them Q (<< 8) and log2 of
+// the run length (<< 16).  Claim c of queue q is tile c % run of run
+// c / run * Q + q.
+__device__ __forceinline__ uint32_t claim_tile(uint32_t* counter, uint32_t queues) {
+    auto* a = (__attribute__((address_space(1))) uint32_t*)counter;
+    const uint32_t c = __hip_atomic_fetch_add(a, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint32_t sh = queues >> 16, run = c >> sh;
+    return ((run * ((queues >> 8) & 0xffu) + (queues & 0xffu)) << sh) + (c - (run << sh));
 }
 
 // A pointer argument of a class function (the same in every lane, which the
@@ -47,74 +65,78 @@ __device__ __forceinline__ const V* uniform_const(const V* p) {
 // the register allocation of the kernel would be the worst path's, and the
 // whole persistent kernel would run at one wave per SIMD.  A call boundary
 // waits for every outstanding memory operation, so a class function keeps
-// claiming tiles while they are of its own class (tiles are sorted by cost,
+// running tiles while they are of its own class (tiles are sorted by cost,
 // so a class comes in runs): the stores of one tile stay in flight while the
 // next tile loads.  It returns the first claimed tile of another class (or
 // past the end).
 template <class Body>
 __device__ __forceinline__ uint32_t tile_run(const BatchTile* __restrict__ tiles, uint32_t ntiles,
-                                             uint32_t* counter, const OpDesc* __restrict__ ops, uint32_t t,
-                                             Body&& body) {
+                                             uint32_t* counter, uint32_t queues, const OpDesc* __restrict__ ops,
+                                             uint32_t t, Body&& body) {
     t = __builtin_amdgcn_readfirstlane(t);
     ntiles = __builtin_amdgcn_readfirstlane(ntiles);
     tiles = uniform_const(tiles);
     ops = uniform_const(ops);
+    uint32_t slot = t >> 31;
+    t &= ~kSlotBit;
     const uint32_t cls = tiles[t].cls;
     for (;;) {
         const BatchTile tl = tiles[t];
         body(ops[tl.arg], tl.g0);
-        __syncthreads();  // the next tile reuses LDS
-        t = claim_tile(counter);
-        if (t >= ntiles || tiles[t].cls != cls) return t;
+        if (threadIdx.x == 0) s_next[slot] = claim_tile(counter, queues);
+        __syncthreads();  // s_next[slot] is written, and the next tile reuses LDS
+        t = __builtin_amdgcn_readfirstlane(s_next[slot]);
+        slot ^= 1;
+        if (t >= ntiles || tiles[t].cls != cls) return t | (slot << 31);
     }
 }
 
 #define MIFFT_TILE_ARGS const BatchTile *__restrict__ tiles, uint32_t ntiles, uint32_t *counter, \
-                        const OpDesc *__restrict__ ops, unsigned char *smem, uint32_t t
-#define MIFFT_TILE_PASS tiles, ntiles, counter, ops, smem, t
+                        uint32_t queues, const OpDesc *__restrict__ ops, unsigned char *smem, uint32_t t
+#define MIFFT_TILE_PASS tiles, ntiles, counter, queues, ops, smem, t
 
 template <class K>
 __device__ __noinline__ uint32_t reg_tiles(MIFFT_TILE_ARGS) {
-    return tile_run(tiles, ntiles, counter, ops, t, [&](const OpDesc& d, uint32_t g0) {
+    return tile_run(tiles, ntiles, counter, queues, ops, t, [&](const OpDesc& d, uint32_t g0) {
         K::tile(d.a, reinterpret_cast<cpx<typename K::T>*>(smem), g0);
     });
 }
 template <class Fmt, int LDM, int STM, bool POST>
 __device__ __noinline__ uint32_t lds_tiles(MIFFT_TILE_ARGS) {
-    return tile_run(tiles, ntiles, counter, ops, t, [&](const OpDesc& d, uint32_t g0) {
+    return tile_run(tiles, ntiles, counter, queues, ops, t, [&](const OpDesc& d, uint32_t g0) {
         lds_fft_tile<Fmt, LDM, STM, POST>(d.a, d.sc, smem, g0);
     });
 }
 template <class Fmt, bool POST>
 __device__ __noinline__ uint32_t mix_tiles(MIFFT_TILE_ARGS) {
-    return tile_run(tiles, ntiles, counter, ops, t, [&](const OpDesc& d, uint32_t g0) {
+    return tile_run(tiles, ntiles, counter, queues, ops, t, [&](const OpDesc& d, uint32_t g0) {
         mix_tile<Fmt, LD_COMPLEX, ST_COMPLEX, POST>(d.a, d.mix, smem, g0);
     });
 }
 template <class Fmt, bool RADER>
 __device__ __noinline__ uint32_t mix_conv_tiles(MIFFT_TILE_ARGS) {
-    return tile_run(tiles, ntiles, counter, ops, t,
+    return tile_run(tiles, ntiles, counter, queues, ops, t,
                     [&](const OpDesc& d, uint32_t g0) { mix_conv_tile<Fmt, RADER>(d.conv, smem, g0); });
 }
 template <bool C2R>
 __device__ __noinline__ uint32_t mix_real_tiles(MIFFT_TILE_ARGS) {
-    return tile_run(tiles, ntiles, counter, ops, t,
+    return tile_run(tiles, ntiles, counter, queues, ops, t,
                     [&](const OpDesc& d, uint32_t g0) { mix_real_tile<C2R>(d.a, d.mix, smem, g0); });
 }
 template <class Fmt, bool MED = false>
 __device__ __noinline__ uint32_t rader_tiles(MIFFT_TILE_ARGS) {
-    return tile_run(tiles, ntiles, counter, ops, t,
+    return tile_run(tiles, ntiles, counter, queues, ops, t,
                     [&](const OpDesc& d, uint32_t g0) { rader_tile<Fmt, MED>(d.conv, smem, g0); });
 }
 template <class K>
 __device__ __noinline__ uint32_t regb_tiles(MIFFT_TILE_ARGS) {
-    return tile_run(tiles, ntiles, counter, ops, t, [&](const OpDesc& d, uint32_t g0) {
+    return tile_run(tiles, ntiles, counter, queues, ops, t, [&](const OpDesc& d, uint32_t g0) {
         K::tile(d.conv, reinterpret_cast<cpx<typename K::T>*>(smem), g0);
     });
 }
 template <class Fmt>
 __device__ __noinline__ uint32_t bluestein_tiles(MIFFT_TILE_ARGS) {
-    return tile_run(tiles, ntiles, counter, ops, t,
+    return tile_run(tiles, ntiles, counter, queues, ops, t,
                     [&](const OpDesc& d, uint32_t g0) { bluestein_tile<Fmt>(d.conv, smem, g0); });
 }
 
@@ -136,7 +158,7 @@ __device__ __forceinline__ void elt_tile(const ConvArgs& c, uint32_t g0) {
 }
 template <class Fmt, int KIND>
 __device__ __noinline__ uint32_t elt_tiles(MIFFT_TILE_ARGS) {
-    return tile_run(tiles, ntiles, counter, ops, t,
+    return tile_run(tiles, ntiles, counter, queues, ops, t,
                     [&](const OpDesc& d, uint32_t g0) { elt_tile<Fmt, KIND>(d.conv, g0); });
 }
 
@@ -146,11 +168,17 @@ __device__ __noinline__ uint32_t elt_tiles(MIFFT_TILE_ARGS) {
 // Up to four workgroups per CU (a launch's LDS is the largest of its tiles,
 // at most 80 KiB: two per CU then): at most 128 VGPRs per lane.
 __global__ void __launch_bounds__(256, 4) k_batch(const BatchTile* __restrict__ tiles, uint32_t ntiles,
-                                               uint32_t* counter, const OpDesc* __restrict__ ops) {
+                                               uint32_t* counter, uint32_t queues,
+                                               const OpDesc* __restrict__ ops) {
     extern __shared__ __align__(16) unsigned char smem[];
-    uint32_t t = claim_tile(counter);
-    while (t < ntiles) {  // uniform: every wave of the block leaves together
-        switch (tiles[t].cls) {
+    const uint32_t q = blockIdx.x % ((queues >> 8) & 0xffu);
+    counter += q * kBatchQueueStride;
+    queues |= q;
+    if (threadIdx.x == 0) s_next[0] = claim_tile(counter, queues);
+    __syncthreads();
+    uint32_t t = __builtin_amdgcn_readfirstlane(s_next[0]) | kSlotBit;
+    while ((t & ~kSlotBit) < ntiles) {  // uniform: every wave of the block leaves together
+        switch (tiles[t & ~kSlotBit].cls) {
             case BC_LDS: t = lds_tiles<FmtF32, LD_COMPLEX, ST_COMPLEX, false>(MIFFT_TILE_PASS); break;
             case BC_LDS_POST: t = lds_tiles<FmtF32, LD_COMPLEX, ST_COMPLEX, true>(MIFFT_TILE_PASS); break;
             case BC_LDS_R2C: t = lds_tiles<FmtF32, LD_REAL, ST_PACKED, false>(MIFFT_TILE_PASS); break;
@@ -215,25 +243,34 @@ __global__ void __launch_bounds__(256, 4) k_batch(const BatchTile* __restrict__ 
             case BC_REGB_2048: t = regb_tiles<RegB2048>(MIFFT_TILE_PASS); break;
             case BC_REGB_4096: t = regb_tiles<RegB4096>(MIFFT_TILE_PASS); break;
             case BC_REGB_8192: t = regb_tiles<RegB8192>(MIFFT_TILE_PASS); break;
-            default: t = claim_tile(counter); break;  // unknown class: skip the tile
+            default: t = tile_run(tiles, ntiles, counter, queues, ops, t, [](const OpDesc&, uint32_t) {}); break;  // unknown class: skip
         }
     }
 }
 
-__global__ void k_batch_reset(uint32_t* counters, uint32_t n) {
-    if (threadIdx.x < n) counters[threadIdx.x] = 0u;
+__global__ void k_batch_reset(uint32_t* counters) {
+    counters[threadIdx.x * kBatchQueueStride] = 0u;
 }
 
-hipError_t launch_batch(const BatchTile* tiles, uint32_t ntiles, uint32_t* counter, const OpDesc* ops,
-                        uint32_t grid, size_t lds_bytes, hipStream_t s) {
+hipError_t launch_batch(const BatchTile* tiles, uint32_t ntiles, uint32_t* counters, uint32_t phase,
+                        const OpDesc* ops, uint32_t grid, size_t lds_bytes, hipStream_t s) {
     hipError_t e = ensure_lds_attr((const void*)&k_batch, lds_bytes);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_batch, dim3(grid), dim3(256), lds_bytes, s, tiles, ntiles, counter, ops);
+    // (fewer workgroups than queues: one queue holds every tile)
+    uint32_t queues = (grid < kBatchQueues ? 1 : kBatchQueues) << 8;
+    // runs of up to 32 tiles (two 65536-point transforms' passes), where every
+    // queue still gets 64 of them (2529 transforms of 127 points, 633 tiles: 22
+    // us one by one, 35 in runs of 32)
+    uint32_t shift = 5;
+    while (shift && (ntiles >> shift) < 64 * kBatchQueues) shift--;
+    queues |= shift << 16;
+    hipLaunchKernelGGL(k_batch, dim3(grid), dim3(256), lds_bytes, s, tiles, ntiles,
+                       counters + phase * kBatchQueues * kBatchQueueStride, queues, ops);
     return hipGetLastError();
 }
 
-hipError_t launch_batch_reset(uint32_t* counters, uint32_t n, hipStream_t s) {
-    hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3(64), 0, s, counters, n);
+hipError_t launch_batch_reset(uint32_t* counters, hipStream_t s) {
+    hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3(kMaxPhases * kBatchQueues), 0, s, counters);
     return hipGetLastError();
 }
 

@@ -175,7 +175,7 @@ static void prepare(mifft_server& S, const mifft_server_request* reqs, int32_t n
             sl.desc_cap = desc_cap;
             hip_check(hipMalloc(&sl.desc, desc_cap), "server descriptors");
             hip_check(hipHostMalloc(&sl.staging, desc_cap, hipHostMallocDefault), "server staging");
-            hip_check(hipMalloc(&sl.counters, 64), "server counters");
+            hip_check(hipMalloc(&sl.counters, kBatchCounterBytes), "server counters");
         }
         hip_check(hipStreamCreateWithFlags(&S.seq_stream, hipStreamNonBlocking), "sequential stream");
     }
