@@ -65,6 +65,10 @@ struct BatchBuild {
 // Appends the entries' ops and tiles to `out`, binding workspace inside
 // [ws_base, ws_base + growth of out.ws_bytes).  Tiles are sorted by cost.
 void batch_build(const BatchEntry* e, int32_t count, char* ws_base, BatchBuild& out);
+// Workspace bytes one entry takes in a batch: its plan's, up to a multiple of
+// kBatchWsPad, and kBatchWsPad more for its start within a 128-byte line.
+constexpr uint64_t kBatchWsPad = 128;
+uint64_t batch_ws_bytes(const Plan& p, uint64_t mult);
 // Device descriptor bytes (ops and tiles) one entry adds to a batch.
 uint64_t batch_desc_bytes(const Plan& p, uint64_t mult);
 // Persistent workgroups for a given LDS footprint: CUs x workgroups per CU.

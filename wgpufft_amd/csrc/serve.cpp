@@ -171,7 +171,8 @@ static void prepare(mifft_server& S, const mifft_server_request* reqs, int32_t n
             hip_check(hipStreamCreateWithFlags(&sl.s2, hipStreamNonBlocking), "server stream");
             hip_check(hipEventCreateWithFlags(&sl.ev2, hipEventDisableTiming), "server event");
             sl.ws_cap = std::max(ws_cap, max_plan_ws);
-            hip_check(hipMalloc(&sl.ws, sl.ws_cap), "server workspace");
+            // (the padding of a tick's entries comes on top of what they are admitted for)
+            hip_check(hipMalloc(&sl.ws, sl.ws_cap + (uint64_t)S.max_items * 2 * kBatchWsPad), "server workspace");
             sl.desc_cap = desc_cap;
             hip_check(hipMalloc(&sl.desc, desc_cap), "server descriptors");
             hip_check(hipHostMalloc(&sl.staging, desc_cap, hipHostMallocDefault), "server staging");
