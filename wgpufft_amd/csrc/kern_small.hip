@@ -81,8 +81,7 @@ __global__ void __launch_bounds__(1024) k_small_volume(SmallVolArgs v) {
                 // flight together (the sum's order is unchanged)
 #pragma unroll 4
                 for (uint32_t q = 0; q < n; q++) {
-                    const cpx<float> x = ln[q * S], w = wt[e];
-                    acc = mk<float>(fma(-x.y, w.y, fma(x.x, w.x, acc.x)), fma(x.y, w.x, fma(x.x, w.y, acc.y)));
+                    acc = acc + cmul(ln[q * S], wt[e]);
                     e += k;
                     e = e >= n ? e - n : e;
                 }
