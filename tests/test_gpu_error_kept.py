@@ -35,3 +35,23 @@ def test_small_volume_direct_sums_round_once_per_term(n0, n1, volumes):
     torch.cuda.synchronize()
     e = rel_l2(y, torch.fft.fft2(x.to(torch.complex128)))
     assert e <= 1.1 * C * U32 * np.sqrt((n0 + n1) / 2 + 5), e
+
+
+@pytest.mark.parametrize("q", [1, 37, 617, 991])
+def test_f64_split_twiddles_from_the_table(q):
+    """The f64 split of 10^6 points: one point q < 1000 goes through the column
+    pass as ones, so that the output is the pass's twiddle W^(q k1) times three
+    stages of row twiddles.  One product of two table entries per output and the
+    stages err by 1.7 u together; a product carried from output to output adds 3
+    to 5 u over the ten of a butterfly."""
+    n = 1000000
+    x = torch.zeros(n, dtype=torch.complex128, device="cuda")
+    x[q] = 1
+    y = torch.empty_like(x)
+    plan = FftPlan.c2c(FftConfig.new(n).with_precision(FftPrecision.F64))
+    assert "lds N=1000" in plan.describe() and " nt=" in plan.describe(), plan.describe()
+    plan.execute(x, y)
+    t = (np.arange(n, dtype=np.int64) * q % n).astype(np.longdouble) / n * 2 * np.arccos(np.longdouble(-1))
+    got = y.cpu().numpy()
+    e = np.sqrt(np.mean((got.real - np.cos(t)) ** 2 + (got.imag + np.sin(t)) ** 2))
+    assert e <= 2.4 * U64, float(e / U64)
