@@ -152,8 +152,9 @@ __device__ __forceinline__ void mix_mid(const Mix& mx, const MixStage& st, const
     }
 }
 
-// The last stage: LDS -> memory, outputs k = j + i n / R.
-template <class Fmt, int STM, bool POST, int R, int NB>
+// The last stage: LDS -> memory, outputs k = j + i n / R.  SCALE: times a.scale
+// (half-length C2R lines were scaled with their bin pairs).
+template <class Fmt, int STM, bool POST, int R, int NB, bool SCALE = true>
 __device__ __forceinline__ void mix_last(const LineArgs& a, const Mix& mx, const MixStage& st,
                                          const cpx<typename Fmt::T>* src, uint32_t g0) {
     using T = typename Fmt::T;
@@ -174,15 +175,17 @@ __device__ __forceinline__ void mix_last(const LineArgs& a, const Mix& mx, const
             const LineBase lb = line_base(a, g);
             const uint32_t o0 = lb.out + at[q].j * (uint32_t)a.out_sk, sk = st.nr * (uint32_t)a.out_sk;
             PostSeq ps;
-            // (f64: a factor of its own per output; carried from output to output
-            // its error grows, 5.4e-16 -> 6.3e-16 over a line of 10^6 points)
+            // (f64: a factor of its own per output, 82.6 -> 87.1 us for five lines of
+            // 10^6 points; carried from output to output its error grows, 5.3e-16 ->
+            // 6.3e-16 over such a line)
             if constexpr (POST && sizeof(T) == 4) ps.init(a, lb.j, at[q].j, st.nr);
 #pragma unroll
             for (int i = 0; i < R; i++) {
                 cpx<T> v = w[q][i];
                 if constexpr (POST && sizeof(T) == 4) v = cmul(v, ps.template next<T>());
                 else if constexpr (POST) v = cmul(v, post_twiddle<T>(a, (uint64_t)lb.j * (at[q].j + i * st.nr)));
-                store_point_at<Fmt, STM, false>(a, o0 + i * sk, lb.j, at[q].j + i * st.nr, mx.n, v);
+                if constexpr (SCALE) store_point_at<Fmt, STM, false>(a, o0 + i * sk, lb.j, at[q].j + i * st.nr, mx.n, v);
+                else Fmt::st(a.out, o0 + i * sk, conj_by(v, sign_mask(a.conj_out)));
             }
         }
     }
@@ -242,7 +245,10 @@ __device__ __forceinline__ void mix_tile(const LineArgs& a, const Mix& mx, unsig
 //   Z[k] = E + i O,  Z[n-k] = conj E + i conj O,
 //   E = X[k] + conj X[n-k],  O = (X[k] - conj X[n-k]) conj W
 // (the imaginary parts of bins 0 and n are dropped).  Half the points go
-// through the stages, and the pairs k, n - k meet in LDS in natural order:
+// through the stages, and the pairs k, n - k meet in LDS in natural order,
+// joined and scaled (C2R: split and scaled) in 64 bits and rounded once (in 32
+// bits 48000 x 400 R2C err 1.06e-7 instead of 9.9e-8, a 1920-point C2R line
+// 1.25e-7 instead of 1.08e-7; R2C takes the same time, C2R 3 to 8 % more):
 // one exchange more than a complex line of n points, where the full-length
 // form runs N0-point lines whose upper half it drops.  48000 x 400 R2C 118 ->
 // 44 us (154 MB, 3.5 TB/s; 30 us at the copy rate), 1920x1080x3 R2C + C2R 127
@@ -294,29 +300,31 @@ constexpr uint32_t kMixPairs = 4;
 template <class T>
 __device__ __forceinline__ void mix_pairs_out(const LineArgs& a, const Mix& mx, const cpx<T>* z, uint32_t g0) {
     const uint32_t n = mx.n, total = mx.lpw * mx.pairs;
-    const T sc = T(0.5) * (T)a.scale;  // the halves of A and B (exact)
+    const double sc = 0.5 * a.scale;  // the halves of A and B (exact)
     for (uint32_t t0 = threadIdx.x; t0 < total; t0 += blockDim.x) {
         const uint32_t lg = mix_div(t0, mx.dpairs), k = t0 - lg * mx.pairs, g = g0 + lg;
         if (g >= a.lines) return;
-        const cpx<T> w = ld_tw<T>(a.half_tw, k);
+        const cpx<double> w = ld_tw<double>(a.half_tw, k);
         const cpx<T>* zl = z + lg * mx.lstr;
-        const cpx<T> p = zl[k], q = zl[k ? n - k : 0];
-        const cpx<T> A = mk<T>(p.x + q.x, p.y - q.y), B = mk<T>(p.y + q.y, q.x - p.x);
-        // A +- W B with two roundings per component
-        const cpx<T> u = mk<T>(fma(-w.y, B.y, fma(w.x, B.x, A.x)), fma(w.y, B.x, fma(w.x, B.y, A.y)));
-        const cpx<T> v = mk<T>(fma(w.y, B.y, fma(-w.x, B.x, A.x)), fma(-w.y, B.x, fma(-w.x, B.y, A.y)));
+        const cpx<T> zp = zl[k], zq = zl[k ? n - k : 0];
+        const cpx<double> p = mk<double>(zp.x, zp.y), q = mk<double>(zq.x, zq.y);
+        const cpx<double> A = mk<double>(p.x + q.x, p.y - q.y), B = mk<double>(p.y + q.y, q.x - p.x);
+        // A +- W B
+        const double wbx = fma(w.x, B.x, -(w.y * B.y)), wby = fma(w.x, B.y, w.y * B.x);
         const uint32_t o = line_base(a, g).out;
-        FmtF32::st(a.out, o + k, mk<T>(u.x * sc, u.y * sc));
-        if (2 * k != n) FmtF32::st(a.out, o + n - k, mk<T>(v.x * sc, -v.y * sc));
+        FmtF32::st(a.out, o + k, mk<T>((T)((A.x + wbx) * sc), (T)((A.y + wby) * sc)));
+        if (2 * k != n) FmtF32::st(a.out, o + n - k, mk<T>((T)((A.x - wbx) * sc), (T)((wby - A.y) * sc)));
     }
 }
 
-// C2R: packed bins -> LDS, conjugated (the inverse is conj DFT conj).
+// C2R: packed bins -> LDS, scaled and conjugated (the inverse is conj DFT conj).
 template <class T>
 __device__ __forceinline__ void mix_pairs_in(const LineArgs& a, const Mix& mx, cpx<T>* z, uint32_t g0) {
     const uint32_t n = mx.n, total = mx.lpw * mx.pairs;
+    const double sc = a.scale;
     for (uint32_t t0 = threadIdx.x; t0 < total; t0 += blockDim.x * kMixPairs) {
-        cpx<T> p[kMixPairs], q[kMixPairs], w[kMixPairs];
+        cpx<T> p[kMixPairs], q[kMixPairs];
+        cpx<double> w[kMixPairs];
         uint32_t lg[kMixPairs], k[kMixPairs];
 #pragma unroll
         for (uint32_t u = 0; u < kMixPairs; u++) {
@@ -326,19 +334,20 @@ __device__ __forceinline__ void mix_pairs_in(const LineArgs& a, const Mix& mx, c
             const uint32_t g = g0 + lg[u], o = line_base(a, g < a.lines ? g : a.lines - 1).in;
             p[u] = FmtF32::ld_c(a.in, o + k[u]);
             q[u] = FmtF32::ld_c(a.in, o + n - k[u]);
-            w[u] = ld_tw<T>(a.half_tw, k[u]);
+            w[u] = ld_tw<double>(a.half_tw, k[u]);
         }
 #pragma unroll
         for (uint32_t u = 0; u < kMixPairs; u++) {
             if (t0 + u * blockDim.x >= total) break;
             if (k[u] == 0) p[u].y = q[u].y = T(0);
-            const cpx<T> E = mk<T>(p[u].x + q[u].x, p[u].y - q[u].y), D = mk<T>(p[u].x - q[u].x, p[u].y + q[u].y);
-            const T wx = w[u].x, wy = w[u].y;
-            // E + i O and conj E + i conj O with O = D conj W, conjugated
+            const cpx<double> P = mk<double>(p[u].x, p[u].y), Q = mk<double>(q[u].x, q[u].y);
+            const cpx<double> E = mk<double>(P.x + Q.x, P.y - Q.y), D = mk<double>(P.x - Q.x, P.y + Q.y);
+            const double wx = w[u].x, wy = w[u].y;
+            const double ox = fma(wx, D.x, wy * D.y), oy = fma(wx, D.y, -(wy * D.x));  // O = D conj W
+            // E + i O and conj E + i conj O, conjugated
             cpx<T>* zl = z + lg[u] * mx.lstr;
-            zl[k[u]] = mk<T>(fma(wy, D.x, fma(-wx, D.y, E.x)), -fma(wy, D.y, fma(wx, D.x, E.y)));
-            if (k[u] && 2 * k[u] != n)
-                zl[n - k[u]] = mk<T>(fma(-wy, D.x, fma(wx, D.y, E.x)), fma(-wy, D.y, fma(-wx, D.x, E.y)));
+            zl[k[u]] = mk<T>((T)((E.x - oy) * sc), (T)((-E.y - ox) * sc));
+            if (k[u] && 2 * k[u] != n) zl[n - k[u]] = mk<T>((T)((E.x + oy) * sc), (T)((E.y - ox) * sc));
         }
     }
 }
@@ -386,7 +395,7 @@ __device__ __forceinline__ void mix_real_tile(const LineArgs& a, const Mix& mx, 
     if constexpr (C2R) {
         switch (st.code) {
 #define MIFFT_MIX_CASE(R, NB) \
-    case R + 32 * NB: mix_last<FmtF32, ST_COMPLEX, false, R, NB>(a, mx, st, src, g0); break;
+    case R + 32 * NB: mix_last<FmtF32, ST_COMPLEX, false, R, NB, false>(a, mx, st, src, g0); break;
             MIFFT_MIX_RADICES(MIFFT_MIX_CASE)
 #undef MIFFT_MIX_CASE
             default: break;

@@ -576,14 +576,14 @@ struct Builder {
         return t;
     }
 
-    // W_n^k for k <= n / 4 (the bin pairs of half-length real lines), f32.
+    // W_n^k for k <= n / 4 (the bin pairs of half-length real lines), f64.
     const void* half_twiddles(uint64_t n) {
         const std::string key = "h" + std::to_string(n);
         auto it = tw_cache.find(key);
         if (it != tw_cache.end()) return it->second;
         const uint64_t cnt = n / 4 + 1;
-        void* t = alloc(cnt * sizeof(cpx<float>), "roots prec=f32 n=" + std::to_string(n) + " count=" + std::to_string(cnt));
-        hip_check(gen_twiddles(P_F32, t, n, cnt, s), "half-length twiddles");
+        void* t = alloc(cnt * sizeof(cpx<double>), "roots prec=f64 n=" + std::to_string(n) + " count=" + std::to_string(cnt));
+        hip_check(gen_twiddles(P_F64, t, n, cnt, s), "half-length twiddles");
         tw_cache[key] = t;
         return t;
     }
