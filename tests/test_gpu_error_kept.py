@@ -88,3 +88,13 @@ def test_half_length_lines_err_as_their_transform_and_one_rounding(kind, n):
     plan, e, (e_half, _) = line_errors(kind, n, (1 << 21) // n)
     assert "half" in plan.describe(), plan.describe()
     assert e <= 1.02 * np.hypot(e_half, C * U32), e / np.hypot(e_half, C * U32)
+
+
+@pytest.mark.parametrize("n", [64, 128, 256, 512])
+def test_compiled_c2r_lines_err_less_than_complex_lines(n):
+    """A full-length inverse of Hermitian bins spreads its error over the real
+    and the imaginary part, which is dropped: 0.87 to 0.9 of a complex line's
+    error, where a half-length transform has all of it (0.95 to 0.98)."""
+    plan, e, (_, e_c2c) = line_errors("c2r", n, (1 << 21) // n)
+    assert plan.describe().startswith("reg "), plan.describe()
+    assert e <= 0.93 * e_c2c, e / e_c2c

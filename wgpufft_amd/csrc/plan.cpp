@@ -844,13 +844,10 @@ struct Builder {
             if (!rv) rv = find_reg_variant(P.prec, (int)n, ld_lf, st_lf, ldm, stm, post, 1);
             if (rv) rv = sized_variant(rv, n, ls.lines, ld_lf, st_lf, ldm, stm, post, pairable);
         }
-        // C2R lines of up to 512 points run at half length (runtime_schedule):
-        // the register kernel reads every packed point twice and transforms
-        // the full length (131072 x 64 points 34.9 against 16.6 us, 32768 x
-        // 256 22.2 against 15.2, 16384 x 512 22.6 against 15.0, few lines
-        // equal; from 1024 points few lines are faster in the register
-        // kernel, 2048 x 1024 7.4 against 9.2 us at 2048 points)
-        if (!tuned && ldm == LD_HERMITIAN && n <= 512 && ls.S1 == 1 && ls.S2 == 1) rv = nullptr;
+        // (C2R lines of compiled lengths keep the full-length register kernel:
+        // at half length (runtime_schedule) large batches are faster, 131072 x
+        // 64 points 34.9 against 16.6 us, but 2 to 3 Mi points of 256 and 512 are
+        // 10 to 30 % slower, and the error is 7 to 14 % larger.)
         const size_t es = elem_bytes(P.arith);
         const uint64_t lstr = lds_line_stride((uint32_t)std::min<uint64_t>(n, 1u << 30));
         if (rv && P.batch_mode && batch_class_for(rv) < 0) rv = nullptr;
