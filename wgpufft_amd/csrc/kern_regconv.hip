@@ -7,6 +7,7 @@ namespace mifft {
 hipError_t ensure_lds_attr(const void* fn, size_t bytes);
 
 #define REGB(K, RADSTR) {K::kM, K::kTPL, K::kLines, K::NT, K::lds_bytes(), (const void*)&reg_bluestein_kernel<K>, RADSTR}
+#define REGB4(K, RADSTR) {K::kM, K::kTPL, K::kLines, K::NT, K::lds_bytes(), (const void*)&reg_bluestein_kernel_w4<K>, RADSTR}
 
 static const RegConvVariant kRegBluestein[] = {
     {RegB8192W::kM, RegB8192W::kTPL, RegB8192W::kLines, RegB8192W::NT, RegB8192W::lds_bytes(),
@@ -16,8 +17,8 @@ static const RegConvVariant kRegBluestein[] = {
     REGB(RegB256, "16x16"),
     REGB(RegB512, "8x8x8"),
     REGB(RegB1024, "16x4x16"),
-    REGB(RegB2048, "16x8x16"),
-    REGB(RegB4096, "16x16x16"),
+    REGB4(RegB2048, "16x8x16"),
+    REGB4(RegB4096, "16x16x16"),
     REGB(RegB8192, "8x16x8x8"),
 };
 

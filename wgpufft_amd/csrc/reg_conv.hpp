@@ -169,6 +169,17 @@ __global__ void __launch_bounds__(K::NT) reg_bluestein_kernel(ConvArgs c) {
     K::run(c, reinterpret_cast<cpx<typename K::T>*>(smem_raw));
 }
 
+// The same at four waves per SIMD, no fewer and no more: unbounded, the 2048-
+// and 4096-point forms take 131 and 130 registers and lose the fourth wave
+// (6482 lines of 647 points 51.5 -> 58.5 us), and a launch bound of four waves
+// trades loads in flight for registers nothing needs (64 lines of 1031 points
+// 8.5 -> 12.0 us).
+template <class K>
+__global__ void __launch_bounds__(K::NT) __attribute__((amdgpu_waves_per_eu(4, 4))) reg_bluestein_kernel_w4(ConvArgs c) {
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    K::run(c, reinterpret_cast<cpx<typename K::T>*>(smem_raw));
+}
+
 // The same with at least MINB waves per SIMD (the register budget that lets
 // two 512-thread workgroups share a CU).
 template <class K, int MINB>
