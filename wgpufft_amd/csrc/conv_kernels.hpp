@@ -24,6 +24,10 @@
 
 namespace mifft {
 
+// Primes above this stage their lines through LDS in natural order; shorter
+// ones (a few cache lines each) gather straight from memory.
+constexpr uint32_t kRaderStagedMin = 64;
+
 // Rader's filter step on the forward spectra in LDS: keeps bin 0 (the sum
 // of the permuted inputs) in s0 and leaves swap(A[k] F[k]) for the inverse.
 template <class T>
@@ -53,14 +57,19 @@ __device__ __forceinline__ void rader_tile(const ConvArgs& c, unsigned char* sme
     cpx<T>* bufB = bufA + lpw * lstr;
     cpx<T>* x0 = bufB + lpw * lstr;  // lpw entries
     cpx<T>* s0 = x0 + lpw;           // lpw entries
-    // Long lines (MED): the line in natural order into bufB (coalesced loads),
+    // Long lines: the line in natural order into bufB (coalesced loads),
     // then the gather a[q] = x[g^q] (zero-padded to M) and x0 = x[0] from
     // LDS, so that no global load waits on the permutation table's.  Short
     // lines (a few cache lines each) gather straight from memory.  Lines
     // past the end read the last line and are never stored.
     const uint32_t total = lpw * M;
+    // (MED: every such prime is longer, but the choice is made at run time: with
+    // the staged form alone, the compiler spills the stages' registers otherwise
+    // and the 128-register kernel is 5 to 6 % slower, 6842 lines of 613 points
+    // 89.0 -> 93.6 us, 2098 of 1999 86.0 -> 92.0)
     const uint32_t tpl = slot_tpl(lpw), slots = tpl * lpw;
-    if constexpr (MED) {
+    const bool staged = MED && p > kRaderStagedMin;
+    if (staged) {
         for (uint32_t s = threadIdx.x; s < slots; s += blockDim.x) {
             const LineSlot m = line_slot(s, lpw, tpl, sc.ld_lf);
             const uint32_t g = g0 + m.l;
@@ -140,7 +149,7 @@ __device__ __forceinline__ void rader_tile(const ConvArgs& c, unsigned char* sme
     // X[g^-u] = x0 + c[u], X[0] = x0 + sum a.  Long lines: permuted in LDS
     // (into the buffer the second transform did not end in), then stored in
     // natural order (coalesced); short lines: scattered straight to memory.
-    if constexpr (MED) {
+    if (staged) {
         cpx<T>* y = (r2 == bufA) ? bufB : bufA;
         for (uint32_t e = threadIdx.x; e < lpw * p; e += blockDim.x) {
             const uint32_t l = fdiv(e, c.dn);
