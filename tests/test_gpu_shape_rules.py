@@ -1,0 +1,20 @@
+"""Which registered shape a pass of power-of-two lines takes, on both sides of
+the lines that the rules draw."""
+import pytest
+
+from wgpufft_amd import FftConfig, FftPlan
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("kind,n,points,pipelined", [
+    ("r2c", 512, 4 << 20, False), ("r2c", 1024, 4 << 20, False), ("r2c", 2048, 4 << 20, False),
+    ("c2r", 1024, 4 << 20, False), ("c2r", 2048, 4 << 20, False),
+    ("r2c", 512, 6 << 20, True), ("r2c", 1024, 6 << 20, True), ("r2c", 2048, 6 << 20, True),
+    ("c2r", 1024, 6 << 20, True), ("c2r", 2048, 6 << 20, True),
+    ("r2c", 256, 4 << 20, False), ("r2c", 256, 8 << 20, True), ("r2c", 256, 32 << 20, False),
+    ("r2c", 4096, 32 << 20, True)])
+def test_real_lines_are_pipelined_where_it_pays(torch_cuda, kind, n, points, pipelined):
+    cfg = (FftConfig.new(n) if kind == "r2c" else FftConfig.inverse(n)).with_batch(points // n)
+    plan = getattr(FftPlan, kind)(cfg)
+    assert ("pipe" in plan.describe()) == pipelined, plan.describe()

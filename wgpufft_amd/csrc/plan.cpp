@@ -650,9 +650,17 @@ struct Builder {
         // 1024 x 4096 10.9 -> 11.3, 2048 x 1024 no better than two lines per
         // workgroup.
         // Real lines gain the same way (R2C of 8192 x 1024 points 18.0 ->
-        // 15.2, of 8192 x 2048 39.4 -> 28.5; C2R 22.5 -> 19.5 and 42.1 -> 33.1).
+        // 15.2, of 8192 x 2048 39.4 -> 28.5; C2R 22.5 -> 19.5 and 42.1 -> 33.1),
+        // but only from 5 Mi points on, where the pass outlasts the fill of its
+        // pipeline: 6 Mi points of 512, 1024 and 2048 R2C 7, 12 and 9 % faster
+        // (C2R of 1024 and 2048 7 and 9), 4 Mi points 4, 11 and 6 % slower (C2R
+        // 4); and 256-point ones up to 24 Mi points (16 Mi 23.8 -> 23.3 us, 32 Mi
+        // 44.6 -> 49.1).
+        const uint64_t points = n * lines;
+        const bool real = ldm != LD_COMPLEX || stm != ST_COMPLEX;
+        const bool pipe = !real || (points >= 5u << 20 && (n > 256 || points <= 24u << 20));
         const RegVariant* best = nullptr;
-        if (P.prec == P_F32)
+        if (P.prec == P_F32 && pipe)
             for (const RegVariant* v : same)
                 if (v->persist && tiles(v) >= 8 * cus && (!best || v->lines < best->lines)) best = v;
         if (best) return best;
