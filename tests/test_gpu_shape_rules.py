@@ -18,3 +18,14 @@ def test_real_lines_are_pipelined_where_it_pays(torch_cuda, kind, n, points, pip
     cfg = (FftConfig.new(n) if kind == "r2c" else FftConfig.inverse(n)).with_batch(points // n)
     plan = getattr(FftPlan, kind)(cfg)
     assert ("pipe" in plan.describe()) == pipelined, plan.describe()
+
+
+@pytest.mark.parametrize("n,columns,shape", [
+    (4096, 512, "vec=1 lpw=4"), (4096, 1024, "vec=1 lpw=4"), (4096, 2048, "vec=2 lpw=8"), (4096, 1025, "vec=1 lpw=4"),
+    (2048, 2048, "vec=2 lpw=8"), (2048, 1025, "vec=1 lpw=8"), (2048, 2049, "vec=1 lpw=4"), (2048, 3880 + 1, "vec=1 lpw=8"),
+    (1024, 1024, "vec=2 lpw=8"), (1024, 2049, "vec=1 lpw=8")])
+def test_column_tiles(torch_cuda, n, columns, shape):
+    """Tiles that have a CU to themselves: 8 lines of 4096 points, or of 2048 one
+    by one (columns of an odd count)."""
+    plan = FftPlan.c2c(FftConfig.new_nd([columns, n]).with_axes([1]))
+    assert shape in plan.describe(), plan.describe()

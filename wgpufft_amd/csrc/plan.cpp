@@ -701,6 +701,13 @@ struct Builder {
     // second CU the tile halves until that is reached (288 columns of 1024
     // points: 12.3, 11.5 and 11.1 us at 8, 4 and 2; 1056 columns are faster
     // at 8 than at 4).
+    // A tile of 8 lines of 4096 points, or of 8 of 2048 one by one, has a CU to
+    // itself.  4096-point lines take it when it fills every CU (2048 columns in
+    // pairs 46.0 -> 37.6 us; 1024 columns 21.0 at 4 lines against 24.6), lone
+    // 2048-point ones unless its last round would be less than half full
+    // (2049 columns, 257 workgroups: 24.0 at 4 against 28.3; 3880 columns, 485:
+    // 37.7 against 36.0).  Pairs halve the waves of a tile: below 8 lines they
+    // go one by one (512 columns of 4096 points 16.0 -> 15.4).
     const RegVariant* strided_variant(const RegVariant* rv, const std::vector<const RegVariant*>& same, uint64_t n,
                                       uint64_t lines, bool ld_lf, int post) {
         const bool columns = ld_lf && !post;
@@ -716,11 +723,14 @@ struct Builder {
         } else {
             want = n >= 256 || (post && n == 128) ? 8 : 32;
         }
-        while (want > 1 && 2 * ((lines + want - 1) / want) < device_cu_count()) want /= 2;
+        const uint64_t cus = device_cu_count();
+        auto tiles = [&](uint64_t per) { return (lines + per - 1) / per; };
+        while (want > 1 && tiles(want) < (n >= 4096 ? cus : (cus + 1) / 2)) want /= 2;
+        if (n == 2048 && want == 8 && rv->vec == 1 && tiles(8) > cus && (tiles(8) - 1) % cus + 1 < cus / 2) want = 4;
         // the widest shape of at most `want` lines, pairs first; else the narrowest
         const RegVariant *best = nullptr, *narrow = nullptr;
         for (const RegVariant* v : same) {
-            if (v->persist) continue;
+            if (v->persist || (v->vec == 2 && v->lines < 8)) continue;
             if (v->lines <= (int)want &&
                 (!best || v->lines > best->lines || (v->lines == best->lines && v->vec > best->vec)))
                 best = v;
