@@ -2,7 +2,7 @@
 the lines that the rules draw."""
 import pytest
 
-from wgpufft_amd import FftConfig, FftPlan
+from wgpufft_amd import FftConfig, FftPlan, FftPrecision
 
 pytestmark = pytest.mark.gpu
 
@@ -29,3 +29,13 @@ def test_column_tiles(torch_cuda, n, columns, shape):
     by one (columns of an odd count)."""
     plan = FftPlan.c2c(FftConfig.new_nd([columns, n]).with_axes([1]))
     assert shape in plan.describe(), plan.describe()
+
+
+@pytest.mark.parametrize("n,lines,f64,tile", [(41, 64, False, 8), (41, 300, False, 8), (29, 300, False, 9), (71, 64, False, 4),
+                                              (211, 64, False, 4), (74, 64, True, 1)])
+def test_few_convolution_lines_spread(torch_cuda, n, lines, f64, tile):
+    """Short of two workgroups per CU a tile takes no more lines than a wave has
+    threads for their butterflies."""
+    cfg = FftConfig.new(n).with_batch(lines).with_precision(FftPrecision.F64 if f64 else FftPrecision.F32)
+    desc = FftPlan.c2c(cfg).describe()
+    assert " nt=" in desc and int(desc.split("lpw=")[1].split()[0]) <= tile, desc

@@ -125,13 +125,15 @@ static double shape_score(int arith, const Mix& x, uint64_t lines, bool lf) {
 }
 
 static double best_shape(int arith, uint64_t n, const std::vector<int>& rad, uint64_t lines, bool ld_lf, bool st_lf,
-                         size_t budget, uint32_t fixed_nt, uint32_t forced_lpw, bool pp, bool real, Mix* out) {
+                         size_t budget, uint32_t fixed_nt, uint32_t forced_lpw, bool pp, bool real, Mix* out,
+                         uint32_t max_lpw = 64) {
     static const uint32_t threads[] = {64, 128, 192, 256, 320, 384, 448, 512, 640, 768, 1024};
     const bool lf = ld_lf || st_lf;
     double best = -1;
     for (uint32_t nt : threads) {
         if (fixed_nt && nt != fixed_nt) continue;
-        for (uint32_t lpw = forced_lpw ? forced_lpw : 1; lpw <= (forced_lpw ? forced_lpw : 64); lpw = lf && !forced_lpw ? 2 * lpw : lpw + 1) {
+        for (uint32_t lpw = forced_lpw ? forced_lpw : 1; lpw <= (forced_lpw ? forced_lpw : max_lpw);
+             lpw = lf && !forced_lpw ? 2 * lpw : lpw + 1) {
             if ((lpw > lines && lpw > 1 && !forced_lpw) || (uint64_t)lpw * n > 0xFFFFu) break;
             // (more than two rounds of 16 points per thread, or under two
             // points: never the best shape)
@@ -234,11 +236,20 @@ bool mix_conv_plan(int arith, uint64_t m, uint64_t lines, bool ld_lf, bool st_lf
     const std::vector<int> rad = mix_schedule(m);
     if (rad.size() < 2 || !lines) return false;
     const std::vector<int> rev(rad.rbegin(), rad.rend());
+    // Few lines: a tile crosses LDS some ten times, and a wave with many short
+    // lines only waits longer at each.  Short of two workgroups per CU a tile
+    // takes the lines whose butterflies are one a thread of a wave, not more (300
+    // lines of 41 points: 10.1 us at 24 lines, f64 64 lines of 74 points 11.6 at 5
+    // and 10.0 at 1).  Batched tiles share the chip with other transforms'.
+    const uint64_t fill = lines / (2ull * device_cu_count());
+    const uint64_t wave = 64 * (uint64_t)*std::min_element(rad.begin(), rad.end()) / m;
+    const uint32_t max_lpw =
+        fixed_nt ? 64 : (uint32_t)std::min<uint64_t>(64, std::max<uint64_t>({1, fill, wave}));
     for (int pp = 0; pp < 2; pp++)
         for (size_t b : {fixed_nt ? budget / 2 : budget, budget}) {
             Mix f;
             // (the two extra elements per line fit what a pitch above m leaves)
-            if (best_shape(arith, m, rad, lines, ld_lf, st_lf, b - 2048, fixed_nt, 0, pp, true, &f) <= 0) continue;
+            if (best_shape(arith, m, rad, lines, ld_lf, st_lf, b - 2048, fixed_nt, 0, pp, true, &f, max_lpw) <= 0) continue;
             Mix r = shape(m, rev, f.lpw, f.nt, ld_lf, st_lf, true);
             if (r.pp && !pp) continue;
             f.lstr = r.lstr = std::max(f.lstr, r.lstr);
