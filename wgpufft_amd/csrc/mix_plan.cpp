@@ -87,6 +87,9 @@ size_t mix_lds_bytes(int arith, const Mix& x) {
     return (size_t)(x.pp ? 2 : 1) * x.lpw * x.lstr * (arith == P_F32 ? 8 : 16);
 }
 
+// Factor of the threads of a workgroup in shape_score: its upper bound too.
+static double thread_score(uint32_t nt) { return nt <= 256 ? 1.0 : nt < 512 ? 0.80 : nt == 512 ? 0.78 : 0.68; }
+
 // Relative rate of a tile shape, 1 at best.  Fitted to 8 Mi-point passes of
 // 15 lengths from 60 to 7680 points, f32 and f64, contiguous and strided,
 // over every thread count: the best contiguous shapes are one to a few lines
@@ -106,7 +109,7 @@ static double shape_score(int arith, const Mix& x, uint64_t lines, bool lf) {
         slots += w * rounds * nb * x.nt;
     }
     double score = useful / slots;
-    score *= x.nt <= 256 ? 1.0 : x.nt < 512 ? 0.80 : x.nt == 512 ? 0.78 : 0.68;
+    score *= thread_score(x.nt);
     // threads resident on a CU hide the barriers and the memory latency of one
     // another (82 registers in f32, 128 to 158 in f64)
     const double reg_threads = arith == P_F32 ? 1280 : 1024;
@@ -131,7 +134,7 @@ static double best_shape(int arith, uint64_t n, const std::vector<int>& rad, uin
     const bool lf = ld_lf || st_lf;
     double best = -1;
     for (uint32_t nt : threads) {
-        if (fixed_nt && nt != fixed_nt) continue;
+        if ((fixed_nt && nt != fixed_nt) || thread_score(nt) <= best) continue;
         for (uint32_t lpw = forced_lpw ? forced_lpw : 1; lpw <= (forced_lpw ? forced_lpw : max_lpw);
              lpw = lf && !forced_lpw ? 2 * lpw : lpw + 1) {
             if ((lpw > lines && lpw > 1 && !forced_lpw) || (uint64_t)lpw * n > 0xFFFFu) break;
@@ -181,30 +184,43 @@ std::vector<int> mix_schedule(uint64_t n) {
     static std::mutex mu;
     static std::map<uint64_t, std::vector<int>> done;  // at most the smooth lengths up to 2^15
     if (n < 2 || n > 0x8000u) return {};
-    std::lock_guard<std::mutex> g(mu);
-    auto f = done.find(n);
-    if (f != done.end()) return f->second;
+    {
+        std::lock_guard<std::mutex> g(mu);
+        auto f = done.find(n);
+        if (f != done.end()) return f->second;
+    }
+    // (searched outside the lock: other threads build plans meanwhile, and two
+    // that search one length find the same)
     std::vector<std::pair<double, std::vector<int>>> sets;
     std::vector<int> cur, best;
     double least = 1e30;
     multisets(n, 16, 0, cur, least, sets);
+    std::stable_sort(sets.begin(), sets.end(), [](const auto& a, const auto& b) { return a.first < b.first; });
     double value = 1e30;
     for (auto& s : sets) {
-        if (s.first > 1.3 * least) continue;
+        if (s.first > 1.3 * least || s.first >= value) continue;  // (a rate is at most 1)
         std::vector<int> r = s.second;
         std::sort(r.begin(), r.end());
+        // The orders of one set differ in the LDS pitch (every stage but the last)
+        // and in which stages must fit one round (every stage but the first and
+        // the last): a rate holds for all orders with those two.
+        double rate[17][17] = {};
         do {
-            double score = r.size() < 2 ? 1.0
-                                        : best_shape(P_F32, n, r, 1u << 30, false, false, kLdsBudget, 0, 0, false,
-                                                     false, nullptr);
-            if (score <= 0) score = 1e-3;
-            const double v = s.first / score * (r.front() < r.back() ? 1.02 : 1.0) * (r.front() < r[r.size() > 1] ? 1.01 : 1.0);
+            double& known = rate[r.front()][r.back()];
+            if (!known) {
+                known = r.size() < 2 ? 1.0
+                                     : best_shape(P_F32, n, r, 1u << 30, false, false, kLdsBudget, 0, 0, false, false,
+                                                  nullptr);
+                if (known <= 0) known = 1e-3;
+            }
+            const double v = s.first / known * (r.front() < r.back() ? 1.02 : 1.0) * (r.front() < r[r.size() > 1] ? 1.01 : 1.0);
             if (v < value) {
                 value = v;
                 best = r;
             }
         } while (std::next_permutation(r.begin(), r.end()));
     }
+    std::lock_guard<std::mutex> g(mu);
     done[n] = best;
     return best;
 }
