@@ -271,6 +271,7 @@ static std::string trim(const std::string& x) {
 
 static bool valid_choice(const std::string& c) {
     if (c.rfind("reg:", 0) == 0) return find_reg_variant_named(c) != nullptr;
+    if (c == "lds:auto") return true;
     if (c.rfind("lds:lpw=", 0) == 0) {
         const std::string v = c.substr(8);
         if (v.empty() || v.size() > 4 || v.find_first_not_of("0123456789") != std::string::npos) return false;
@@ -844,6 +845,8 @@ struct Builder {
                 rv = t;
                 tuned = true;
             }
+        } else if (choice == "lds:auto") {
+            tuned = true;  // the runtime schedule with the tile it picks itself
         } else if (choice.rfind("lds:lpw=", 0) == 0) {
             forced_lpw = (uint32_t)std::strtoul(choice.c_str() + 8, nullptr, 10);
             tuned = forced_lpw > 0;
@@ -2420,13 +2423,20 @@ int autotune_sequence(const mifft_config* cfgs, const mifft_kind* kinds, int cou
                 c.a.tw = TB.stage_twiddles(T.arith, Builder::parse_radices(v->radices));
                 cands.emplace_back(reg_variant_name(v), c);
             }
+            // the runtime schedule: the tile it picks by itself (what an untuned
+            // plan of a length without a compiled variant runs: any line count and
+            // any thread count), and fixed line counts as long as they fit
             const uint64_t lstr = lds_line_stride(ref->n);
             const size_t es = elem_bytes(ref->prec == P_F32 ? P_F32 : P_F64);
-            for (uint32_t lpw = 1; lpw <= 32 && !ref->fold; lpw *= 2) {
-                if (2 * lstr * es * lpw > T.lds_budget || lpw > ref->a.lines) break;
+            if (!ref->fold && 2 * lstr * es <= T.lds_budget) {
                 Op c = *ref;
-                TB.runtime_schedule(c, false, lpw);
-                cands.emplace_back("lds:lpw=" + std::to_string(lpw), c);
+                TB.runtime_schedule(c, false, 0);
+                cands.emplace_back("lds:auto", c);
+                for (uint32_t lpw = 1; lpw <= 32 && lpw <= ref->a.lines; lpw *= 2) {
+                    TB.runtime_schedule(c, false, lpw);
+                    if ((c.mix.ns ? c.mix.lpw : c.sc.lpw) != lpw) break;
+                    cands.emplace_back("lds:lpw=" + std::to_string(lpw), c);
+                }
             }
             if (cands.size() < 2) continue;
             auto apply = [&](const Op& c) {

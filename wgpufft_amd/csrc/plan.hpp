@@ -153,7 +153,7 @@ const Op* plan_launch_op(const Plan& p, int index);
 // Process-wide tuning table: measured line-kernel choices keyed by op shape
 // (precision, length, lane layout, load/store modes, twiddle, pairability,
 // line-count bucket).  A choice is a registered variant name ("reg:...") or
-// a runtime-schedule LDS shape ("lds:lpw=<lines per workgroup>").
+// a runtime schedule ("lds:auto", or "lds:lpw=<lines per workgroup>").
 std::string tuning_lookup(const std::string& key);
 void tuning_set(const std::string& key, const std::string& choice);
 void tuning_clear();
