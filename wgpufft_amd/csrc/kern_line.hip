@@ -307,6 +307,7 @@ static const RegVariant kRegistry[] = {
     // 8192 x 512 16.2 -> 14.6, 32768 x 256 26.5 -> 24.2; 128-point lines lose
     // 2-20 %, strided columns 2-18 %)
     REGP(FmtF32, P_F32, 1024, 64, 2, 0, 0, LD_COMPLEX, ST_COMPLEX, 0, 1, 2, "16x16x4", 16, 16, 4),
+    REGP(FmtF32, P_F32, 1024, 128, 2, 0, 0, LD_COMPLEX, ST_COMPLEX, 0, 1, 2, "8x8x4x4", 8, 8, 4, 4),
     REGP(FmtF32, P_F32, 2048, 128, 1, 0, 0, LD_COMPLEX, ST_COMPLEX, 0, 1, 2, "16x16x8", 16, 16, 8),
     REGP(FmtF32, P_F32, 512, 32, 4, 0, 0, LD_COMPLEX, ST_COMPLEX, 0, 1, 2, "8x8x8", 8, 8, 8),
     REGP(FmtF32, P_F32, 256, 16, 8, 0, 0, LD_COMPLEX, ST_COMPLEX, 0, 1, 2, "16x16", 16, 16),
