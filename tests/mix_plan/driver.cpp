@@ -162,6 +162,12 @@ int main() {
                             EXPECT(x.pairs == n / 2 + 1 && mix_lds_bytes(arith, x) <= budget, "real n=%u", x.n);
                         }
                         MixConv c;
+                        // a convolution that the LDS-to-LDS form would fit (two buffers and
+                        // two points) has a tile: no longer form of it is kept
+                        const size_t es = arith == P_F32 ? 8 : 16;
+                        if (n > 16 && (2 * (size_t)lds_line_stride((uint32_t)n) + 2) * es <= budget)
+                            EXPECT(mix_conv_plan(arith, n, lines, ld, st, budget, fixed, &c), "conv n=%llu has no tile",
+                                   (unsigned long long)n);
                         if (mix_conv_plan(arith, n, lines, ld, st, budget, fixed, &c)) {
                             // (Rader keeps p = n + 1 points in natural order)
                             check_tile("conv", c.f, n, fixed, true, (uint32_t)n + (n % 2 == 0));

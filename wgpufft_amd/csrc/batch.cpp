@@ -49,8 +49,8 @@ static std::string batch_reject_reason(const Plan& p) {
         switch (op->kind) {
             case OP_REG: ok = batch_class_for(op->rv) >= 0; break;
             case OP_LDS: ok = batch_lds_class(op->prec, op->ldm, op->stm, op->post, op->mix.ns > 0) >= 0; break;
+            case OP_BLUESTEIN: ok = op->rcv || op->prec == P_F64; break;
             case OP_RADER:
-            case OP_BLUESTEIN:
             case OP_CHIRP_PRE:
             case OP_POINTWISE:
             case OP_CHIRP_POST: ok = op->prec == P_F32 || op->prec == P_F64; break;
@@ -255,12 +255,10 @@ void batch_build(const BatchEntry* entries, int32_t count, char* ws_base, BatchB
                     break;
                 case OP_RADER:
                 case OP_BLUESTEIN:
-                    if (op.conv.mix)
-                        cls = op.kind == OP_RADER ? (f64 ? BC_MIX_RADER_F64 : BC_MIX_RADER)
-                                                  : (f64 ? BC_MIX_BLUESTEIN_F64 : BC_MIX_BLUESTEIN);
-                    else if (f64) cls = op.kind == OP_RADER ? BC_RADER_F64 : BC_BLUESTEIN_F64;
-                    else if (op.kind == OP_RADER) cls = sched_has_medium_prime(op.conv.sc) ? BC_RADER_MED : BC_RADER;
-                    else cls = BC_BLUESTEIN;
+                    if (op.kind == OP_BLUESTEIN) cls = op.conv.mix ? BC_MIX_BLUESTEIN_F64 : BC_BLUESTEIN_F64;
+                    else if (op.conv.mix) cls = f64 ? BC_MIX_RADER_F64 : BC_MIX_RADER;
+                    else if (f64) cls = BC_RADER_F64;
+                    else cls = sched_has_medium_prime(op.conv.sc) ? BC_RADER_MED : BC_RADER;
                     d.conv = op.conv;
                     if (op.conv.mix) {
                         // a plan made for one line: the tile for all lines that run it

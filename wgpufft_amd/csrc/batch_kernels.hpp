@@ -11,7 +11,6 @@ enum BatchClass : uint32_t {
     BC_LDS = 0,
     BC_LDS_POST,
     BC_RADER,
-    BC_BLUESTEIN,
     BC_REG_C4096,
     BC_REG_C2048,
     BC_REG_C1024,
@@ -69,8 +68,7 @@ enum BatchClass : uint32_t {
     BC_MIX_C2R,
     BC_MIX_RADER,  // convolutions of a runtime schedule (mix_conv.hpp)
     BC_MIX_RADER_F64,
-    BC_MIX_BLUESTEIN,
-    BC_MIX_BLUESTEIN_F64,
+    BC_MIX_BLUESTEIN_F64,  // (f32 Bluestein: the register classes, or passes of their own)
     BC_COUNT
 };
 

@@ -193,10 +193,8 @@ __global__ void __launch_bounds__(256, 4) k_batch(const BatchTile* __restrict__ 
             case BC_MIX_C2R: t = mix_real_tiles<true>(MIFFT_TILE_PASS); break;
             case BC_MIX_RADER: t = mix_conv_tiles<FmtF32, true>(MIFFT_TILE_PASS); break;
             case BC_MIX_RADER_F64: t = mix_conv_tiles<FmtF64, true>(MIFFT_TILE_PASS); break;
-            case BC_MIX_BLUESTEIN: t = mix_conv_tiles<FmtF32, false>(MIFFT_TILE_PASS); break;
             case BC_MIX_BLUESTEIN_F64: t = mix_conv_tiles<FmtF64, false>(MIFFT_TILE_PASS); break;
             case BC_RADER: t = rader_tiles<FmtF32>(MIFFT_TILE_PASS); break;
-            case BC_BLUESTEIN: t = bluestein_tiles<FmtF32>(MIFFT_TILE_PASS); break;
             case BC_RADER_F64: t = rader_tiles<FmtF64>(MIFFT_TILE_PASS); break;
             case BC_RADER_MED: t = rader_tiles<FmtF32, true>(MIFFT_TILE_PASS); break;
             case BC_BLUESTEIN_F64: t = bluestein_tiles<FmtF64>(MIFFT_TILE_PASS); break;

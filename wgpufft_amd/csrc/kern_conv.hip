@@ -52,8 +52,7 @@ hipError_t launch_rader(int prec, const ConvArgs& c, hipStream_t s) {
             if (sched_has_medium_prime(c.sc))
                 return wide ? launch_conv<FmtF32>(k_rader<FmtF32, true, 512>, prec, c, s, 512)
                             : launch_conv<FmtF32>(k_rader_mb<FmtF32, true, 512, 4>, prec, c, s, 512);
-            return wide ? launch_conv<FmtF32>(k_rader<FmtF32, false, 512>, prec, c, s, 512)
-                        : launch_conv<FmtF32>(k_rader<FmtF32>, prec, c, s);
+            return launch_conv<FmtF32>(k_rader<FmtF32>, prec, c, s);  // (at most 16 points: 64 KiB)
         case P_F64:
             return wide ? launch_conv<FmtF64>(k_rader<FmtF64, false, 512>, prec, c, s, 512)
                         : launch_conv<FmtF64>(k_rader<FmtF64>, prec, c, s);
@@ -66,9 +65,7 @@ hipError_t launch_rader(int prec, const ConvArgs& c, hipStream_t s) {
 hipError_t launch_bluestein(int prec, const ConvArgs& c, hipStream_t s) {
     const bool wide = conv_kernel_bytes(prec, c.m, c.sc.lpw) > kLdsBudget / 2;
     switch (prec) {
-        case P_F32:
-            return wide ? launch_conv<FmtF32>(k_bluestein<FmtF32, 512>, prec, c, s, 512)
-                        : launch_conv<FmtF32>(k_bluestein<FmtF32>, prec, c, s);
+        case P_F32: return hipErrorInvalidValue;  // reg_conv.hpp up to 4096 points, mix_conv.hpp above
         case P_F64:
             return wide ? launch_conv<FmtF64>(k_bluestein<FmtF64, 512>, prec, c, s, 512)
                         : launch_conv<FmtF64>(k_bluestein<FmtF64>, prec, c, s);
