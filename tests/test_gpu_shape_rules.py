@@ -2,7 +2,9 @@
 the lines that the rules draw."""
 import pytest
 
+import wgpufft_amd as W
 from wgpufft_amd import FftConfig, FftPlan, FftPrecision
+from wgpufft_amd.tune import DEFAULT_TABLE
 
 pytestmark = pytest.mark.gpu
 
@@ -39,3 +41,21 @@ def test_few_convolution_lines_spread(torch_cuda, n, lines, f64, tile):
     cfg = FftConfig.new(n).with_batch(lines).with_precision(FftPrecision.F64 if f64 else FftPrecision.F32)
     desc = FftPlan.c2c(cfg).describe()
     assert " nt=" in desc and int(desc.split("lpw=")[1].split()[0]) <= tile, desc
+
+
+@pytest.mark.parametrize("shape,axes,batch,kind", [([1024], None, 3072, "c2c"), ([256], None, 32768, "c2c"),
+                                                   ([24576, 256], [1], 1, "c2c"), ([3072, 2048], [1], 1, "c2c"),
+                                                   ([2048], None, 2048, "r2c")])
+def test_committed_table_leaves_better_rules_alone(torch_cuda, shape, axes, batch, kind):
+    """Passes where the built-in rule runs the faster shape (or the same): the
+    committed table holds no choice for them."""
+    cfg = FftConfig.new_nd(shape).with_batch(batch)
+    if axes:
+        cfg = cfg.with_axes(axes)
+    W.clear_tuning()
+    built_in = getattr(FftPlan, kind)(cfg).describe()
+    W.load_tuning(DEFAULT_TABLE)
+    try:
+        assert getattr(FftPlan, kind)(cfg).describe() == built_in
+    finally:
+        W.clear_tuning()
