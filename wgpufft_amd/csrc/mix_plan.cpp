@@ -37,6 +37,13 @@ static uint32_t nb_for(int r, uint32_t need) {
     }
 }
 
+// Whether stage s of ns writes a second buffer: a stage from LDS to LDS that takes
+// more than one round does (the middle ones, and the last (first) one where the
+// bin pairs of real lines follow (precede) it).
+static bool needs_second(bool real, uint32_t s, uint32_t ns, uint32_t need, uint32_t nb) {
+    return (real || (s >= 1 && s + 1 < ns)) && need > nb;
+}
+
 static Mix shape(uint64_t n, const std::vector<int>& rad, uint32_t lpw, uint32_t nt, bool ld_lf, bool st_lf,
                  bool real) {
     Mix x;
@@ -71,10 +78,7 @@ static Mix shape(uint64_t n, const std::vector<int>& rad, uint32_t lpw, uint32_t
         st.dLp = mix_mag(st.Lp);
         if (s >= 1) twoff += (R - 1) * L;
         if (s + 1 < x.ns) x.lstr = std::max(x.lstr, R * st.nrp);
-        // a stage from LDS to LDS that takes more than one round writes a
-        // second buffer: the middle stages, and the last (first) one where the
-        // bin pairs of real lines follow (precede) it
-        if ((real || (s >= 1 && s + 1 < x.ns)) && need > nb) pp = true;
+        pp |= needs_second(real, s, x.ns, need, nb);
         L *= R;
     }
     x.lstr |= 1u;
@@ -90,40 +94,61 @@ size_t mix_lds_bytes(int arith, const Mix& x) {
 // Factor of the threads of a workgroup in shape_score: its upper bound too.
 static double thread_score(uint32_t nt) { return nt <= 256 ? 1.0 : nt < 512 ? 0.80 : nt == 512 ? 0.78 : 0.68; }
 
-// Relative rate of a tile shape, 1 at best.  Fitted to 8 Mi-point passes of
+// What the shapes of one schedule share.
+struct Stages {
+    uint32_t ns, lstr;
+    uint32_t r[kMixStages], nr[kMixStages];
+    double w[kMixStages];  // work of a butterfly
+    Stages(uint64_t n, const std::vector<int>& rad) : ns((uint32_t)rad.size()), lstr(0) {
+        for (uint32_t s = 0; s < ns; s++) {
+            r[s] = (uint32_t)rad[s];
+            nr[s] = (uint32_t)n / r[s];
+            w[s] = butterfly_ops(rad[s]) + 8.0 * rad[s];
+            if (s + 1 < ns) lstr = std::max(lstr, r[s] * (nr[s] | 1u));
+        }
+        lstr |= 1u;
+    }
+};
+
+// Relative rate of a tile shape, 1 at best; 0 where it does not fit `budget`, or
+// needs a second buffer and may not (pp) have one.  Fitted to 8 Mi-point passes of
 // 15 lengths from 60 to 7680 points, f32 and f64, contiguous and strided,
 // over every thread count: the best contiguous shapes are one to a few lines
 // in 64 to 256 threads (1080 points: 1 line, 128 threads 28.5 us; 4 lines,
 // 512 threads 33.3 us; 576 threads 45 us), since a barrier then holds up few
 // waves; more than 256 threads cost 10 to 30 %, most where they are not a
 // multiple of the four SIMDs' waves.
-static double shape_score(int arith, const Mix& x, uint64_t lines, bool lf) {
-    const size_t es = arith == P_F32 ? 8 : 16, lds = mix_lds_bytes(arith, x);
+static double shape_score(int arith, const Stages& st, uint32_t lpw, uint32_t nt, uint64_t lines, bool lf, size_t budget,
+                          bool pp, bool real) {
+    const size_t es = arith == P_F32 ? 8 : 16;
     // share of the launched lanes' butterfly slots that do work
     double useful = 0, slots = 0;
-    for (uint32_t s = 0; s < x.ns; s++) {
-        const uint32_t R = x.st[s].code & 31u, nb = x.st[s].code >> 5, total = x.lpw * x.st[s].nr;
-        const double w = butterfly_ops((int)R) + 8.0 * R;
-        const uint32_t rounds = (total + x.nt * nb - 1) / (x.nt * nb);
-        useful += w * total;
-        slots += w * rounds * nb * x.nt;
+    bool second = false;
+    for (uint32_t s = 0; s < st.ns; s++) {
+        const uint32_t total = lpw * st.nr[s], need = (total + nt - 1) / nt, nb = nb_for((int)st.r[s], need);
+        const uint32_t rounds = (total + nt * nb - 1) / (nt * nb);
+        second |= needs_second(real, s, st.ns, need, nb);
+        useful += st.w[s] * total;
+        slots += st.w[s] * rounds * nb * nt;
     }
+    const size_t lds = (size_t)(second ? 2 : 1) * lpw * st.lstr * es;
+    if (lds > budget || (second && !pp)) return 0;
     double score = useful / slots;
-    score *= thread_score(x.nt);
+    score *= thread_score(nt);
     // threads resident on a CU hide the barriers and the memory latency of one
     // another (82 registers in f32, 128 to 158 in f64)
     const double reg_threads = arith == P_F32 ? 1280 : 1024;
-    const double wgs_cu = std::floor(std::min((double)kLdsBudget / (double)lds, std::max(1.0, reg_threads / x.nt)));
-    score *= std::sqrt(std::min(1.0, wgs_cu * x.nt / 1024.0));
+    const double wgs_cu = std::floor(std::min((double)kLdsBudget / (double)lds, std::max(1.0, reg_threads / nt)));
+    score *= std::sqrt(std::min(1.0, wgs_cu * nt / 1024.0));
     // strided sides: the row segment of a tile; neighbouring tiles run on the
     // same XCD and share what is left of a line through its L2
     if (lf) {
-        const size_t seg = x.lpw * es;
+        const size_t seg = lpw * es;
         score *= seg >= 128 ? 1.0 : seg >= 64 ? 0.97 : seg >= 32 ? 0.9 : seg >= 16 ? 0.7 : 0.4;
     }
     // at least two workgroups per CU where the lines allow it
-    const double wgs = std::ceil((double)lines / x.lpw), want = 2.0 * device_cu_count();
-    if (wgs < want && x.lpw > 1) score *= 0.3 + 0.7 * wgs / want;
+    const double wgs = std::ceil((double)lines / lpw), want = 2.0 * device_cu_count();
+    if (wgs < want && lpw > 1) score *= 0.3 + 0.7 * wgs / want;
     return score;
 }
 
@@ -132,7 +157,9 @@ static double best_shape(int arith, uint64_t n, const std::vector<int>& rad, uin
                          uint32_t max_lpw = 64) {
     static const uint32_t threads[] = {64, 128, 192, 256, 320, 384, 448, 512, 640, 768, 1024};
     const bool lf = ld_lf || st_lf;
+    const Stages st(n, rad);
     double best = -1;
+    uint32_t best_lpw = 0, best_nt = 0;
     for (uint32_t nt : threads) {
         if ((fixed_nt && nt != fixed_nt) || thread_score(nt) <= best) continue;
         for (uint32_t lpw = forced_lpw ? forced_lpw : 1; lpw <= (forced_lpw ? forced_lpw : max_lpw);
@@ -142,15 +169,16 @@ static double best_shape(int arith, uint64_t n, const std::vector<int>& rad, uin
             // points: never the best shape)
             if (!fixed_nt && !forced_lpw && lpw > 1 && (uint64_t)lpw * n > 34ull * nt) break;
             if (!fixed_nt && !forced_lpw && nt > 64 && (uint64_t)lpw * n < 2ull * nt) continue;
-            const Mix x = shape(n, rad, lpw, nt, ld_lf, st_lf, real);
-            if (mix_lds_bytes(arith, x) > budget || (x.pp && !pp)) break;
-            const double score = shape_score(arith, x, lines, lf);
+            const double score = shape_score(arith, st, lpw, nt, lines, lf, budget, pp, real);
+            if (score <= 0) break;
             if (score > best + 1e-9) {
                 best = score;
-                if (out) *out = x;
+                best_lpw = lpw;
+                best_nt = nt;
             }
         }
     }
+    if (out && best > 0) *out = shape(n, rad, best_lpw, best_nt, ld_lf, st_lf, real);
     return best;
 }
 
