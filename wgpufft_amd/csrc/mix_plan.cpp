@@ -94,6 +94,13 @@ size_t mix_lds_bytes(int arith, const Mix& x) {
 // Factor of the threads of a workgroup in shape_score: its upper bound too.
 static double thread_score(uint32_t nt) { return nt <= 256 ? 1.0 : nt < 512 ? 0.80 : nt == 512 ? 0.78 : 0.68; }
 
+// Factor of the workgroups, at least two per CU where the lines allow it: falls
+// with the lines of a workgroup.
+static double fill_score(uint64_t lines, uint32_t lpw) {
+    const double wgs = std::ceil((double)lines / lpw), want = 2.0 * device_cu_count();
+    return wgs < want && lpw > 1 ? 0.3 + 0.7 * wgs / want : 1.0;
+}
+
 // What the shapes of one schedule share.
 struct Stages {
     uint32_t ns, lstr;
@@ -146,10 +153,7 @@ static double shape_score(int arith, const Stages& st, uint32_t lpw, uint32_t nt
         const size_t seg = lpw * es;
         score *= seg >= 128 ? 1.0 : seg >= 64 ? 0.97 : seg >= 32 ? 0.9 : seg >= 16 ? 0.7 : 0.4;
     }
-    // at least two workgroups per CU where the lines allow it
-    const double wgs = std::ceil((double)lines / lpw), want = 2.0 * device_cu_count();
-    if (wgs < want && lpw > 1) score *= 0.3 + 0.7 * wgs / want;
-    return score;
+    return score * fill_score(lines, lpw);
 }
 
 static double best_shape(int arith, uint64_t n, const std::vector<int>& rad, uint64_t lines, bool ld_lf, bool st_lf,
@@ -169,6 +173,7 @@ static double best_shape(int arith, uint64_t n, const std::vector<int>& rad, uin
             // points: never the best shape)
             if (!fixed_nt && !forced_lpw && lpw > 1 && (uint64_t)lpw * n > 34ull * nt) break;
             if (!fixed_nt && !forced_lpw && nt > 64 && (uint64_t)lpw * n < 2ull * nt) continue;
+            if (!forced_lpw && thread_score(nt) * fill_score(lines, lpw) <= best) break;  // nor any wider tile
             const double score = shape_score(arith, st, lpw, nt, lines, lf, budget, pp, real);
             if (score <= 0) break;
             if (score > best + 1e-9) {
