@@ -27,8 +27,9 @@ namespace mifft {
 // 128-byte lines that both touch (transforms start at any 16 bytes).  And
 // device atomics on one address are served one at a time, some 6 ns each.
 // Tiles are sorted by cost, so the queues hold equal work.  One counter and no
-// runs against this, by itself: 2047 transforms of 65536 points 1236 -> 1121
-// us, 2329 of 4096 63 -> 56, 2172 of 1001 40 -> 31, 2485 of 343 22 -> 15.
+// runs against this, a length by itself (17 to 19 transforms of 1 to 256 lines):
+// 2047 lines of 65536 points 1236 -> 1121 us, 2329 of 4096 63 -> 56, 2172 of
+// 1001 40 -> 31, 2485 of 343 22 -> 15.
 // (Claiming the next tile before the current one's loads, to hide the atomic,
 // measured 1221: the in-order memory counter makes the loads wait for it.)
 //
@@ -257,8 +258,8 @@ hipError_t launch_batch(const BatchTile* tiles, uint32_t ntiles, uint32_t* count
     // (fewer workgroups than queues: one queue holds every tile)
     uint32_t queues = (grid < kBatchQueues ? 1 : kBatchQueues) << 8;
     // runs of up to 32 tiles (two 65536-point transforms' passes), where every
-    // queue still gets 64 of them (2529 transforms of 127 points, 633 tiles: 22
-    // us one by one, 35 in runs of 32)
+    // queue still gets 64 of them (18 transforms, 2529 lines of 127 points, 633
+    // tiles: 22 us one by one, 35 in runs of 32)
     uint32_t shift = 5;
     while (shift && (ntiles >> shift) < 64 * kBatchQueues) shift--;
     queues |= shift << 16;

@@ -65,7 +65,7 @@ hipError_t launch_lds(int prec, int ldm, int stm, int post, const LineArgs& a, c
 size_t lds_kernel_bytes(int prec, uint32_t n, uint32_t lpw);
 constexpr size_t kLdsBudget = 160 * 1024;
 
-// Runtime-schedule register line kernels (mix_kernels.hpp, kern_mix.hip): the
+// Runtime-schedule register line kernels (mix_kernels.hpp, kern_mix_*.hip): the
 // schedule and tile shape of one length (mix_plan.cpp).  Counts are in
 // elements; the d* fields are mix_div multipliers.
 constexpr int kMixStages = 6;  // enough for every length up to 2^15

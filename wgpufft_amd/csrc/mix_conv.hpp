@@ -8,10 +8,11 @@
 // S-stage lines crosses LDS 2 S - 2 times (plus Rader's two permutations),
 // where the LDS-to-LDS form crosses it 4 S + 4 times and keeps two buffers.
 // Bound by those exchanges and the vector units (1009 points: two transforms
-// of 1008 points per line).  us per pass, LDS-to-LDS -> this: 8192 lines of
-// 1009 points 99 -> 54 (2.5 TB/s), 65536 of 127 100 -> 47, 2^18 of 31 125 -> 55,
-// 4096 of 2003 120 -> 60, 1000 of 7561 143 -> 91, f64 4096 of 1009 97 -> 59,
-// f64 Bluestein 4096 of 611 103 -> 73.
+// of 1008 points per line).  us per pass, LDS-to-LDS -> this, over one pair of
+// arrays: 8192 lines of 1009 points 99 -> 54 (three pairs in turn, beyond the
+// last-level cache: 99.7 -> 61.4, 2.2 TB/s), 65536 of 127 100 -> 47, 2^18 of 31
+// 125 -> 55, 4096 of 2003 120 -> 60, 1000 of 7561 143 -> 91, f64 4096 of 1009
+// 97 -> 59, f64 Bluestein 4096 of 611 103 -> 73.
 #pragma once
 #include "conv_kernels.hpp"
 #include "mix_kernels.hpp"

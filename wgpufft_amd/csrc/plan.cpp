@@ -453,8 +453,10 @@ static bool adjacent_lines(const LineSet& ls, const Layout& l) {
 
 // Estimated cost per point of one four-step pass over lines of length n:
 // register-resident kernels stream at close to the copy rate; runtime-
-// schedule LDS lines run well when many fit a workgroup (short lines) and
-// poorly when only a few do (long f64 lines: narrow strided row segments).
+// schedule lines run well when many fit a workgroup (short lines) and poorly
+// when only a few do (long f64 lines: narrow strided row segments).  The counts
+// are those of the two-buffer form (lds_fft_kernel) whose passes these costs
+// were fitted to; the one-buffer register form that runs them now holds more.
 static double pass_cost(int prec, uint64_t n) {
     if (n <= (1u << 30) && !find_reg_variants(prec, (int)n, 1, 1, LD_COMPLEX, ST_COMPLEX, 1).empty()) return 1.0;
     const size_t es = prec == P_F32 ? 8 : 16;
@@ -464,7 +466,7 @@ static double pass_cost(int prec, uint64_t n) {
 }
 
 // Best four-step split n = n1 * n2 (both smooth, both on chip under
-// `budget`) by estimated cost, ties broken toward balance; 0 if none.
+// `budget`, counted with two buffers) by estimated cost, ties broken toward balance; 0 if none.
 static uint64_t best_split(int prec, uint64_t n, size_t budget, double* cost_out) {
     uint64_t best1 = 0;
     double best = 1e30;
