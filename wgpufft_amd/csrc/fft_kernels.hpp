@@ -696,11 +696,19 @@ struct RegFft {
         cpx<T> fa[VEC], fb[VEC];
         load_lines(a, t0 * LINES, wa, fa);
         uint32_t i = 0;
-        for (; i + 2 < nt; i += 2) {
-            load_lines(a, (t0 + (i + 1) * G) * LINES, wb, fb);
-            stage<0, false>(a, lds, (t0 + i * G) * LINES, wa, twr, fa);
-            load_lines(a, (t0 + (i + 2) * G) * LINES, wa, fa);
-            stage<0, false>(a, lds, (t0 + (i + 1) * G) * LINES, wb, twr, fb);
+        // A do loop, which is rotated as it stands: the compiler left the for loop's
+        // head, which every tile's first loads were awaited in, in place (1024-point
+        // lines 229 registers instead of 220, 256-point ones 202 instead of 170, a
+        // spill at 4096; 4096 lines of 1024 points, beyond the cache, 15.5 us
+        // instead of 15.0).
+        if (nt > 2) {
+            do {
+                load_lines(a, (t0 + (i + 1) * G) * LINES, wb, fb);
+                stage<0, false>(a, lds, (t0 + i * G) * LINES, wa, twr, fa);
+                load_lines(a, (t0 + (i + 2) * G) * LINES, wa, fa);
+                stage<0, false>(a, lds, (t0 + (i + 1) * G) * LINES, wb, twr, fb);
+                i += 2;
+            } while (i + 2 < nt);
         }
         if (i + 1 < nt) {
             load_lines(a, (t0 + (i + 1) * G) * LINES, wb, fb);
