@@ -33,6 +33,23 @@ def test_column_tiles(torch_cuda, n, columns, shape):
     assert shape in plan.describe(), plan.describe()
 
 
+@pytest.mark.parametrize("n,batch,shape", [
+    (65536, 64, "N=256 16x16 lines=16384 tpl=16 vec=1 lpw=16"), (65536, 4, "N=256 16x16 lines=1024 tpl=16 vec=1 lpw=8"),
+    (131072, 4, "lpw=8"), (262144, 16, "lpw=16"), (16384, 256, "N=128 16x8 lines=32768 tpl=8 vec=1 lpw=32"),
+    (16384, 128, "N=128 16x8 lines=16384 tpl=8 vec=1 lpw=8")])
+def test_twiddled_columns_tile(torch_cuda, n, batch, shape):
+    """The columns of a two-pass split: 16 lines of 256 and 512 points where that
+    fills every CU, 32 of 128 from four tiles per CU on."""
+    first = FftPlan.c2c(FftConfig.new(n).with_batch(batch)).describe().split(";")[0]
+    assert " post" in first and shape in first, first
+
+
+def test_twiddled_columns_of_one_line(torch_cuda):
+    """4096 columns of 128 points, the middle pass of 2^19: eight lines per tile."""
+    middle = FftPlan.c2c(FftConfig.new(1 << 19)).describe().split(";")[1]
+    assert " post" in middle and "N=128 16x8 lines=4096 tpl=8 vec=1 lpw=8" in middle, middle
+
+
 @pytest.mark.parametrize("n,lines,f64,tile", [(41, 64, False, 8), (41, 300, False, 8), (29, 300, False, 9), (71, 64, False, 4),
                                               (211, 64, False, 4), (74, 64, True, 1)])
 def test_few_convolution_lines_spread(torch_cuda, n, lines, f64, tile):

@@ -687,8 +687,7 @@ struct Builder {
     // (8160 columns of 512 points 27.6 us against 30.4 at 32 and 4;  4128 of
     // 1024 points, in pairs, 30.6 against 34.2 one by one; 2016 of 2048 31.4
     // against 39.1 at 2; 8192 of a 4096 x 2048 fold 16 us less than 16 lines
-    // one by one), 32 for shorter lines, 8 for 128-point lines that store
-    // with a twiddle (32768 of them 27.3 against 28.4 at 32), and
+    // one by one), 32 for shorter lines, and
     // min(16, 4096 / n) for contiguous loads with transposed stores (16384
     // of 512 points 51.5 against 53.4 at 16; 8192 of 1024 59.8 against 61.4;
     // 32 at 64 points: 65536 of them 43.8 against 45.4 at 16).
@@ -700,7 +699,14 @@ struct Builder {
     // 32; 1024-point ones that store with a twiddle 75 against 66 at 16), 96
     // MiB for plain columns of 1024 points and up and transposed stores of
     // 512 and up (1024-point columns of 64 MiB: 58.1 at 8, 59.8 at 16;
-    // 512-point rows of 128 MiB: equal).  Short of a workgroup for every
+    // 512-point rows of 128 MiB: equal).  256- and 512-point columns
+    // that store with a twiddle go at 16 lines where that fills every CU (64 x
+    // 65536 points in place, both directions, 52.2 -> 50.2 us, over arrays that
+    // take turns 59.1 -> 54.1, and 16 x 262144 64.9 -> 58.9; from one array to
+    // another, over and over, 26.0 -> 28.5), at 8 where not (2048 columns
+    // of 256 points 20.7 against 21.5 at 16);  128-point ones at 32 from four
+    // tiles per CU on (256 x 16384 points in place 54.4 -> 52.6, in turns 60.4
+    // -> 57.0), at 8 below (3 x 2^19 points 27.8 -> 26.4).  Short of a workgroup for every
     // second CU the tile halves until that is reached (288 columns of 1024
     // points: 12.3, 11.5 and 11.1 us at 8, 4 and 2; 1056 columns are faster
     // at 8 than at 4).
@@ -724,10 +730,11 @@ struct Builder {
         } else if (!ld_lf) {
             want = n < 128 ? 32 : std::min<uint64_t>(16, std::max<uint64_t>(1, 4096 / n));
         } else {
-            want = n >= 256 || (post && n == 128) ? 8 : 32;
+            want = post && (n == 256 || n == 512) ? 16 : n >= 256 ? 8 : 32;
         }
         const uint64_t cus = device_cu_count();
         auto tiles = [&](uint64_t per) { return (lines + per - 1) / per; };
+        if (ld_lf && post && n >= 128 && want > 8 && tiles(want) < (n == 128 ? 4 * cus : cus)) want = 8;
         while (want > 1 && tiles(want) < (n >= 4096 ? cus : (cus + 1) / 2)) want /= 2;
         if (n == 2048 && want == 8 && rv->vec == 1 && tiles(8) > cus && (tiles(8) - 1) % cus + 1 < cus / 2) want = 4;
         // the widest shape of at most `want` lines, pairs first; else the narrowest
