@@ -50,6 +50,15 @@ def test_twiddled_columns_of_one_line(torch_cuda):
     assert " post" in middle and "N=128 16x8 lines=4096 tpl=8 vec=1 lpw=8" in middle, middle
 
 
+@pytest.mark.parametrize("shape,axes,pipelined", [
+    ([256, 256, 64], None, False), ([256, 256, 128], None, False), ([512, 128, 64], None, False),
+    ([512, 256, 64], None, True), ([1024, 64, 64], None, True), ([256, 256, 64], [0], True), ([512, 128, 64], [0], True)])
+def test_complex_lines_of_several_axes(torch_cuda, shape, axes, pipelined):
+    cfg = FftConfig.new_nd(shape)
+    desc = FftPlan.c2c(cfg.with_axes(axes) if axes else cfg).describe()
+    assert ("pipe" in desc) == pipelined, desc
+
+
 @pytest.mark.parametrize("n,lines,f64,tile", [(41, 64, False, 8), (41, 300, False, 8), (29, 300, False, 9), (71, 64, False, 4),
                                               (211, 64, False, 4), (74, 64, True, 1)])
 def test_few_convolution_lines_spread(torch_cuda, n, lines, f64, tile):

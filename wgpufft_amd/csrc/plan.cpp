@@ -659,9 +659,17 @@ struct Builder {
         // (C2R of 1024 and 2048 7 and 9), 4 Mi points 4, 11 and 6 % slower (C2R
         // 4); and 256-point ones up to 24 Mi points (16 Mi 23.8 -> 23.3 us, 32 Mi
         // 44.6 -> 49.1).
+        // Complex 256- and 512-point lines that are one axis of several: from 6 Mi
+        // points of 512 on (512x256x64 in place 146.1 -> 142.7 for both directions;
+        // 512x128x64 70.8 -> 77.6, 512x100x100 100.7 -> 104.5, so those are not),
+        // 256 never (256x256x64 75.0 -> 85.2, 256x60x400 119.8 -> 125.3, 256x256x96
+        // 109.0 -> 107.7).  Longer ones are the faster out of place (1024x64x64 80.3
+        // -> 76.4, 2048x32x64 84.6 -> 81.6) by more than they lose in place (75.8 ->
+        // 76.9, 78.5 -> 81.0).
         const uint64_t points = n * lines;
         const bool real = ldm != LD_COMPLEX || stm != ST_COMPLEX;
-        const bool pipe = !real || (points >= 5u << 20 && (n > 256 || points <= 24u << 20));
+        const bool pipe = real ? points >= 5u << 20 && (n > 256 || points <= 24u << 20)
+                               : P.cfg.naxes <= 1 || n > 512 || (n == 512 && points >= 6u << 20);
         const RegVariant* best = nullptr;
         if (P.prec == P_F32 && pipe)
             for (const RegVariant* v : same)
