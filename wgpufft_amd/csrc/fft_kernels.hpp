@@ -699,7 +699,7 @@ struct RegFft {
         // A do loop, which is rotated as it stands: the compiler left the for loop's
         // head, which every tile's first loads were awaited in, in place (1024-point
         // lines 229 registers instead of 220, 256-point ones 202 instead of 170, a
-        // spill at 4096; 4096 lines of 1024 points, beyond the cache, 15.5 us
+        // spill at 4096; 4096 lines of 1024 points, beyond the cache, 15.3 us
         // instead of 15.0).
         if (nt > 2) {
             do {
